@@ -2,7 +2,8 @@
 // strided-batched sgemm (rocBLAS on the library's stream) and saxpy (a
 // HIP kernel).  Replaces kernels/src/cuda/Tensor.cu:132-206, whose GEMMs go
 // through cuBLAS with TF32 math on sm >= 80 (runtime.cu:20-24); here every
-// product is computed in fp32 (rocBLAS's fp32 MFMA kernels for gfx950).
+// product is computed in fp32 (rocBLAS's fp32 MFMA kernels for gfx950).  The
+// Linear layers' products run the kernels of gemm_split.hip where those serve.
 //
 // gpt.c's matrices are row-major; rocBLAS is column-major.  A row-major
 // C (M x N) = op(A) op(B) is the column-major C^T (N x M) = op(B)^T op(A)^T,
@@ -19,9 +20,11 @@
 #include <set>
 #include <tuple>
 #include "blas.hpp"
+#include "gemm_split.hpp"
 #include "gemm_tuned.hpp"
 #include "gpu_kernels.h"
 #include "hip_check.hpp"
+#include "ops_common.hpp"
 #include "utils.h"
 
 namespace {
@@ -109,9 +112,9 @@ void gptc_blas_destroy() {
 
 namespace {
 
-// Tuned solutions.  rocBLAS picks a Tensile kernel for a GEMM by a heuristic;
-// for the GEMMs of a GPT-2 small training step that pick runs 5-24 % slower
-// than the fastest solution rocBLAS itself lists for the same problem.  The
+// Tuned solutions of sgemm calls.  rocBLAS picks a Tensile kernel for a GEMM by a
+// heuristic; for the products of a GPT-2 small training step that pick runs 5-24 %
+// slower than the fastest solution rocBLAS itself lists for the same problem.  The
 // table gemm_tuned.inc (written by tune_gemm from a log of the library's own
 // calls, see gemm_tuned.hpp) names that solution per problem.  A listed
 // problem is run with its solution, checked by rocBLAS on first use; a
@@ -230,122 +233,16 @@ void gptc_sgemm(int trans_a, int trans_b, int M, int N, int K, float alpha, cons
     colmajor_gemm(op(trans_b), op(trans_a), N, M, K, alpha, B, ldb, A, lda, beta, C, ldc, "sgemm");
 }
 
-namespace {
-
-// out[i] (+)= p[0][i] + p[1][i] + ... + p[S-1][i], in that order; `accumulate`
-// adds the sum to out, otherwise it overwrites out.
-__global__ __launch_bounds__(kThreads) void add_partials_kernel(const float *__restrict__ p, float *__restrict__ out,
-                                                               int64_t n, int S, bool vec, bool accumulate) {
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-    if (vec) {
-        const int64_t n4 = n / 4;
-        for (int64_t i = blockIdx.x * kThreads + threadIdx.x; i < n4; i += stride) {
-            f32x4 acc = reinterpret_cast<const f32x4 *>(p)[i];
-            for (int s = 1; s < S; ++s) acc += reinterpret_cast<const f32x4 *>(p + s * n)[i];
-            if (accumulate) {
-                f32x4 o = reinterpret_cast<f32x4 *>(out)[i];
-                o += acc;
-                acc = o;
-            }
-            reinterpret_cast<f32x4 *>(out)[i] = acc;
-        }
-    } else {
-        for (int64_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-            float acc = p[i];
-            for (int s = 1; s < S; ++s) acc += p[s * n + i];
-            out[i] = accumulate ? out[i] + acc : acc;
-        }
-    }
-}
-
-void launch_add_partials(const float *partial, float *out, int64_t n, int S, bool accumulate, hipStream_t s) {
-    int64_t blocks = (n / 4 + kThreads - 1) / kThreads;
-    if (blocks > 256 * 8) blocks = 256 * 8;
-    const bool vec = (n % 4) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    add_partials_kernel<<<dim3(static_cast<int>(blocks < 1 ? 1 : blocks)), dim3(kThreads), 0, s>>>(partial, out, n, S,
-                                                                                                   vec, accumulate);
-    hipCheck(hipGetLastError());
-}
-
-}  // namespace
-
-void gptc_sgemm_wgrad(int out_f, int in_f, int rows, const float *g, const float *x, float *dW) {
-    if (out_f <= 0 || in_f <= 0) return;
-    // Output tiles of 128 x 128; below about two per CU rocBLAS's default
-    // pick cannot fill 256 CUs, so the row (K) range is split into S slices
-    // computed as one strided-batched GEMM, and the slices are added in a
-    // fixed order.
-    // A tuned solution for one of the split counts 1, 2, 4, 8 fixes S: the
-    // table holds one per weight gradient, chosen with the slices' add pass
-    // counted (with tuned kernels GPT-2's c_fc and c_proj products fill the
-    // GPU unsplit).
-    const int64_t n_out = static_cast<int64_t>(out_f) * in_f;
-    int S = 0;
-    for (int s = 1; s <= 8 && S == 0; s *= 2) {
-        if (rows % s != 0) continue;
-        const int c = rows / s;
-        const gptc::GemmProblem p =
-            s == 1 ? problem(rocblas_operation_none, rocblas_operation_transpose, in_f, out_f, rows, in_f, out_f, in_f,
-                             0, 0, 0, 0, 1.0f, 1.0f)
-                   : problem(rocblas_operation_none, rocblas_operation_transpose, in_f, out_f, c, in_f, out_f, in_f,
-                             static_cast<long long>(c) * in_f, static_cast<long long>(c) * out_f, n_out, s, 1.0f, 0.0f);
-        if (find_tuned(p) >= 0) S = s;
-    }
-    if (S == 0) {
-        const int64_t tiles = static_cast<int64_t>((out_f + 127) / 128) * ((in_f + 127) / 128);
-        S = 1;
-        while (S < 8 && tiles * S < 512 && rows % (2 * S) == 0 && rows / (2 * S) >= 1024) S *= 2;
-    }
-    if (S == 1) {
-        gptc_sgemm(1, 0, out_f, in_f, rows, 1.0f, g, out_f, x, in_f, 1.0f, dW, in_f);
+void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
+                      const float *bias, const float *add, float *C) {
+    const gptc::SplitGemm g{A, B, C, bias, add, M, N, K, lda, ldb, N, trans_a, trans_b};
+    if (gptc::split_gemm_serves(g)) {
+        gptc::launch_split_gemm(g, gptc_stream_checked());
         return;
     }
-    hipStream_t s = gptc_stream_checked();
-    const int chunk = rows / S;
-    const int64_t n = static_cast<int64_t>(out_f) * in_f;
-    float *partial = static_cast<float *>(alloc_cuda(sizeof(float) * static_cast<size_t>(n) * S));
-    const float one = 1.0f, zero = 0.0f;
-    // Column-major view: partial_b^T (in x out) = x_b^T (in x chunk) g_b (chunk x out).
-    colmajor_gemm_batched(rocblas_operation_none, rocblas_operation_transpose, in_f, out_f, chunk, one, x, in_f,
-                          static_cast<long long>(chunk) * in_f, g, out_f, static_cast<long long>(chunk) * out_f, zero,
-                          partial, in_f, n, S, "sgemm_strided_batched (weight gradient)");
-    launch_add_partials(partial, dW, n, S, true, s);
-    free_cuda(partial);
-}
-
-void gptc_sgemm_dgrad(int rows, int in_f, int out_f, const float *g, const float *W, float *dx) {
-    if (rows <= 0 || in_f <= 0) return;
-    // With rocBLAS's atomics off, a product with few 128 x 128 output tiles and
-    // a long reduction runs on one wave of tiles with a third of the CUs idle
-    // (GPT-2's lm_head input gradient: 384 tiles, K = 50257, 113 TFLOP/s).  The
-    // reduction is then split into S equal slices, as in the weight gradient,
-    // while every slice keeps at least 8192 terms: below that the extra passes
-    // over the slices cost more than the fuller GPU gains (measured at K = 2304
-    // and 3072).  The K - S*chunk leftover terms are added into slice 0.
-    const int64_t tiles = static_cast<int64_t>((rows + 127) / 128) * ((in_f + 127) / 128);
-    int S = 1;
-    while (S < 8 && tiles * S < 512 && out_f / (2 * S) >= 8192) S *= 2;
-    if (S == 1) {
-        gptc_sgemm(0, 0, rows, in_f, out_f, 1.0f, g, out_f, W, in_f, 0.0f, dx, in_f);
-        return;
-    }
-    hipStream_t s = gptc_stream_checked();
-    const int chunk = out_f / S, rest = out_f - S * chunk;
-    const int64_t n = static_cast<int64_t>(rows) * in_f;
-    float *partial = static_cast<float *>(alloc_cuda(sizeof(float) * static_cast<size_t>(n) * S));
-    const float one = 1.0f, zero = 0.0f;
-    // Column-major view: partial_b^T (in x rows) = W_b^T (in x chunk) g_b^T (chunk x rows),
-    // W_b = rows [b*chunk, (b+1)*chunk) of W, g_b = the same columns of g.
-    colmajor_gemm_batched(rocblas_operation_none, rocblas_operation_none, in_f, rows, chunk, one, W, in_f,
-                          static_cast<long long>(chunk) * in_f, g, out_f, chunk, zero, partial, in_f, n, S,
-                          "sgemm_strided_batched (input gradient)");
-    if (rest > 0) {
-        const int64_t k0 = static_cast<int64_t>(S) * chunk;
-        colmajor_gemm(rocblas_operation_none, rocblas_operation_none, in_f, rows, rest, one, W + k0 * in_f, in_f,
-                      g + k0, out_f, one, partial, in_f, "sgemm (input gradient, leftover terms)");
-    }
-    launch_add_partials(partial, dx, n, S, false, s);
-    free_cuda(partial);
+    CHECK_ERROR(add != nullptr && add != C, "gptc_linear_gemm: rocBLAS accumulates into C only.");
+    gptc_sgemm(trans_a, trans_b, M, N, K, 1.0f, A, lda, B, ldb, add != nullptr ? 1.0f : 0.0f, C, N);
+    if (bias != nullptr && M > 0 && N > 0) gptc::launch_bias_add(C, bias, M, N, gptc_stream_checked());
 }
 
 extern "C" void sgemm_cuda(const int TransA, const int TransB, const int M, const int N, const int K,

@@ -2,9 +2,11 @@
 // (Tensile kernel) chosen for it by measurement, for the table gemm_tuned.inc
 // that blas.hip compiles in.
 //
-// The table is regenerated on an MI355X from a log of the problems the
-// library itself issues (so that its keys match the calls exactly):
-//   GPTC_GEMM_LOG=/tmp/gemms.txt python3 bench.py --workload gpt2 --steps 1 --warmup 0 --no-cpu-baseline
+// The table serves the sgemm entry points (the Linear layers run the kernels of
+// gemm_split.hip).  It is regenerated on an MI355X from a log of the rocBLAS
+// problems that a program makes the library issue (so that its keys match the
+// calls exactly):
+//   GPTC_GEMM_LOG=/tmp/gemms.txt <the program>
 //   make -C gpt.c_amd tune && gpt.c_amd/_build/tune_gemm /tmp/gemms.txt > gpt.c_amd/csrc/gemm_tuned.inc
 // tune_gemm (tune_gemm.cpp) times every solution rocBLAS lists for each
 // problem of at least 1 GFLOP, re-times the fastest few, and keeps the winner
@@ -13,11 +15,10 @@
 // a repeat.  Solution indices are those of this image's rocBLAS; another
 // rocBLAS rejects them on first use and the default pick runs instead.
 //
-// Weight gradients: gptc_sgemm_wgrad uses the split count S of a tuned entry
-// when the table has one for its product at S = 1, 2, 4 or 8 (one per
-// product), else its tile-count rule.  Those entries come from a tune_gemm
-// run over the four split counts of each product (log lines written by hand
-// in the format above), the fastest GEMM plus its slices' add pass chosen.
+// The weight gradient entries (op(B) transposed, one per product) come from a
+// tune_gemm run over the split counts 1, 2, 4 and 8 of each product (log lines
+// written by hand in the format above), the fastest GEMM plus its slices' add
+// pass chosen.
 #pragma once
 
 namespace gptc {

@@ -1,12 +1,8 @@
 // Linear layer kernels, y = x W^T + b (replaces kernels/src/cuda/Linear.cu:40-95,
 // semantics of kernels/src/cpu/Linear.c:4-80):
-//   forward   one fp32 GEMM (rocBLAS) then a bias pass over y;
+//   forward   one fp32 product with the bias added as it is written;
 //   backward  dx = g W (overwrites dout), dW += g^T x, db += column sums of g.
-// dW's GEMM has a small output (out x in) and a long reduction (B*T rows):
-// it is split over row slices (one strided-batched GEMM) and the slices are
-// added into dW in a fixed order, so it fills the GPU and stays deterministic.
-// dx's GEMM is split the same way over its reduction (out features) when that
-// is long and the output small: GPT-2's lm_head (K = 50257, 8192 x 768).
+// The products are gptc_linear_gemm's (gemm_split.hip).
 // The column sums are deterministic: workgroups sum fixed row ranges into a
 // partial buffer, and a second kernel adds the partials in a fixed order
 // (the reference uses one atomicAdd per workgroup and column); float4
@@ -231,9 +227,8 @@ extern "C" void linear_forward_cuda_kernel(const tensor_t *W, const tensor_t *b,
         check_gpu(b, "b");
         CHECK_ERROR(b->length != out_f, "Expected b to hold %d elements, but got %d.", out_f, b->length);
     }
-    hipStream_t s = gptc_stream_checked();
-    gptc_sgemm(0, 1, rows, out_f, in_f, 1.0f, input->t, in_f, W->t, in_f, 0.0f, output->t, out_f);
-    if (b != NULL && rows > 0) launch_bias_add(output->t, b->t, rows, out_f, s);
+    gptc_linear_gemm(false, true, rows, out_f, in_f, input->t, in_f, W->t, in_f, b != NULL ? b->t : nullptr, nullptr,
+                     output->t);
 }
 
 extern "C" void linear_backward_cuda_kernel(const tensor_t *global_grad, const tensor_t *cache, const tensor_t *W,
@@ -256,9 +251,9 @@ extern "C" void linear_backward_cuda_kernel(const tensor_t *global_grad, const t
         CHECK_ERROR(db->length != out_f, "Expected db to hold %d elements, but got %d.", out_f, db->length);
     }
     hipStream_t s = gptc_stream_checked();
-    // dx = g W : (rows x out) (out x in), split over out when the reduction is long and the output small
-    gptc_sgemm_dgrad(rows, in_f, out_f, global_grad->t, W->t, dout->t);
-    // dW += g^T x : (out x rows) (rows x in), split over rows when the output is small
-    gptc_sgemm_wgrad(out_f, in_f, rows, global_grad->t, cache->t, dW->t);
+    // dx = g W : (rows x out) (out x in)
+    gptc_linear_gemm(false, false, rows, in_f, out_f, global_grad->t, out_f, W->t, in_f, nullptr, nullptr, dout->t);
+    // dW += g^T x : (out x rows) (rows x in)
+    gptc_linear_gemm(true, false, out_f, in_f, rows, global_grad->t, out_f, cache->t, in_f, nullptr, dW->t, dW->t);
     if (db != NULL) launch_column_sum_add(global_grad->t, db->t, rows, out_f, s);
 }
