@@ -449,8 +449,9 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
                 "The forward kept the log-sum-exp-only state, which only the D = 64 kernels read, but these "
                 "gradient buffers need the other kernels (unaligned rows).");
     hipStream_t s = gptc_stream_checked();
-    float *ds_scratch = nullptr;
-    if (lse_only && p.full) {
+    p.slab = gptc::bwd_slab(p);
+    float *ds_scratch = nullptr, *db_part = nullptr;
+    if (lse_only && p.full && !p.slab) {
         const int64_t bh = static_cast<int64_t>(d.B) * d.H;
         const int64_t per_head = static_cast<int64_t>(gptc::bwd_ds_floats(1, 1, d.T));
         const int64_t heads = std::min<int64_t>(bh, g_scratch_limit.load() / per_head);
@@ -461,7 +462,7 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
             p.ds_heads = static_cast<int>(heads);
         }
     }
-    gptc::bwd_split_plan(p, s);
+    if (!p.slab) gptc::bwd_split_plan(p, s);
     bool folded = false;
     if (bias != nullptr) {
         CHECK_ERROR(!compact, "The qkv bias can be folded in with the compact cache layout only.");
@@ -482,6 +483,11 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
             p.dbq_part = cache[3]->t + st.dbq;
             p.dbkv_part = cache[3]->t + st.dbkv;
             p.C = d.C;
+            if (p.slab) {
+                db_part = static_cast<float *>(
+                    alloc_cuda(static_cast<size_t>(d.B) * gptc::slab_count(p) * 3 * d.C * sizeof(float)));
+                p.dbq_part = db_part;
+            }
         }
     }
     gptc::launch_attn_bwd(p, s, g_have_events ? g_events + 2 : nullptr);
@@ -490,7 +496,10 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
     if (ds_scratch != nullptr) free_cuda(ds_scratch);
     if (bias != nullptr) {
         const int nqt = (d.T + 63) / 64, nkb = (d.T + 127) / 128;
-        if (folded) {
+        if (folded && p.slab) {
+            gptc::launch_add_column_partials(db_part, db->t, d.B * gptc::slab_count(p), 3 * d.C, s);
+            free_cuda(db_part);
+        } else if (folded) {
             // db += the per-block column sums, in a fixed order.
             gptc::launch_add_column_partials(p.dbq_part, db->t, d.B * nqt, d.C, s);
             gptc::launch_add_column_partials(p.dbkv_part, db->t + d.C, d.B * (nkb + p.nsplit), 2 * d.C, s);

@@ -1325,6 +1325,15 @@ size_t bwd_ds_floats(int B, int H, int T) {
 
 void launch_attn_bwd(const BwdParams &p_in, hipStream_t stream, const hipEvent_t *ev) {
     BwdParams p = p_in;
+    if (p.slab) {
+        // One launch, timed as dk/dv.
+        if (ev)
+            for (int i = 0; i < 3; ++i) hipCheck(hipEventRecord(ev[i], stream));
+        launch_attn_bwd_slab(p, stream);
+        if (ev)
+            for (int i = 3; i < 6; ++i) hipCheck(hipEventRecord(ev[i], stream));
+        return;
+    }
     const bool wide = p.D > kDPad;  // 64 < D <= 128: the DP = 128 kernels
     // The 32-row dq kernel for head sizes other than 64, and its grid order
     // (the 16-row one runs work lists).

@@ -976,6 +976,12 @@ void launch_attn_fwd(const FwdParams &p_in, hipStream_t stream, const hipEvent_t
         if (ev) hipCheck(hipEventRecord(ev[1], stream));
         return;
     }
+    if (fwd_slab(p)) {
+        if (ev) hipCheck(hipEventRecord(ev[0], stream));
+        launch_attn_fwd_slab(p, stream);
+        if (ev) hipCheck(hipEventRecord(ev[1], stream));
+        return;
+    }
     if (p.full) {
         // Short heads leave P' to the backward; in the compact layout they
         // run one workgroup per block, in the reference layout the DEEP

@@ -100,6 +100,7 @@ struct BwdParams {
     // heads run in chunks [ds_bh0, ds_bh0 + ds_heads) (ds_bh0 set per chunk
     // by launch_attn_bwd).  ds == nullptr: both gradient kernels recompute P.
     bool lse_only;
+    bool slab;            // the slab kernel runs (bwd_slab)
     int ds_heads;
     int ds_bh0;
 };
@@ -152,6 +153,15 @@ void launch_attn_decode(const DecParams &p, hipStream_t stream);
 // nullptr: no events.
 void launch_attn_fwd(const FwdParams &p, hipStream_t stream, const hipEvent_t *ev);
 void launch_attn_bwd(const BwdParams &p, hipStream_t stream, const hipEvent_t *ev);
+
+// The slab kernels (attn_slab.hip): whether they run a problem, their launches, and the
+// 16-row slabs of a sequence.  The backward is one launch; with the qkv bias
+// folded in (p.db set), p.dbq_part then takes (B * slab_count(p)) x 3C column sums.
+bool fwd_slab(const FwdParams &p);
+bool bwd_slab(const BwdParams &p);
+int slab_count(const BwdParams &p);
+void launch_attn_fwd_slab(const FwdParams &p, hipStream_t stream);
+void launch_attn_bwd_slab(const BwdParams &p, hipStream_t stream);
 
 // Head sizes past 2 * kDPad, up to kGenericMaxD: plain-FMA kernels
 // (attn_generic.hip) with the LSE-only state.  The backward launcher runs

@@ -1,0 +1,54 @@
+"""GPU parity of the slab kernels (csrc/attn_slab.hip) at the edges of their
+blocks, slabs and tiles, against the oracle at the tolerance of
+tests/test_attention_gpu.py, for one and two row blocks per wave, every padded
+head size, and the qkv bias folded in.
+"""
+import numpy as np
+import pytest
+
+import gptc
+from test_attention_gpu import compare_with_oracle
+from test_gpt2_gpu import self_attention_vs_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,T,C,H", [
+    # heads of 64: one block per slab (few tiles), T around blocks, slabs and tiles
+    (1, 15, 64, 1), (1, 16, 64, 1), (2, 17, 128, 2), (1, 64, 128, 2), (1, 65, 128, 2), (2, 128, 256, 4),
+    (1, 129, 64, 1), (1, 143, 128, 2), (1, 144, 64, 1), (1, 145, 64, 1), (2, 192, 128, 2), (1, 193, 64, 1),
+    (1, 321, 192, 3),
+    # two blocks per slab (350 tiles or more)
+    (4, 176, 768, 12), (4, 177, 768, 12), (4, 191, 768, 12), (1, 1024, 192, 3), (1, 1009, 192, 3),
+    # other head sizes: 4, 16, 36, 60 padded to 64, and 68, 80, 124, 128 to 128
+    (2, 33, 8, 2), (1, 100, 16, 1), (2, 70, 72, 2), (3, 200, 120, 2), (2, 48, 136, 2), (2, 161, 160, 2), (1, 97, 248, 2),
+    (1, 640, 512, 4), (8, 200, 512, 4), (2, 512, 96, 3),
+])
+def test_slabs_against_oracle(rt, oracle, B, T, C, H):
+    print(f"case slab B={B} T={T} C={C} H={H}", flush=True)
+    compare_with_oracle(rt, oracle, B, T, C, H)
+
+
+@pytest.mark.parametrize("B,T,C,H", [(1, 40, 128, 2), (2, 129, 128, 2), (1, 333, 192, 3), (4, 177, 768, 12)])
+def test_slabs_with_qkv_bias(rt, oracle, B, T, C, H):
+    """The bias added to the rows and its gradient from the slabs' column sums (one and two blocks per slab)."""
+    print(f"case slab bias B={B} T={T} C={C} H={H}", flush=True)
+    self_attention_vs_oracle(rt, oracle, B, T, C, H)
+
+
+def test_slabs_are_deterministic(rt):
+    """The waves' partial results join in wave order: the same bits on every run."""
+    B, T, C, H = 3, 333, 320, 5
+    x, dy = rt.normal((B, T, 3 * C), 11), rt.normal((B, T, C), 12)
+    seen = []
+    for _ in range(2):
+        layer = gptc.AttentionLayer(rt, C, H, T)
+        layer.to(gptc.CUDA)
+        y = layer.forward(rt.from_numpy(x))
+        y_np = rt.to_numpy(y)
+        d = layer.backward(rt.from_numpy(dy))
+        seen.append((y_np, rt.to_numpy(d)))
+        rt.free(y)
+        rt.free(d)
+        layer.free()
+    assert all(np.array_equal(a, b) for a, b in zip(*seen))
