@@ -233,6 +233,24 @@ void gptc_sgemm(int trans_a, int trans_b, int M, int N, int K, float alpha, cons
     colmajor_gemm(op(trans_b), op(trans_a), N, M, K, alpha, B, ldb, A, lda, beta, C, ldc, "sgemm");
 }
 
+namespace {
+
+// y[i incy] += alpha x[i incx], i < n.
+void launch_saxpy(int64_t n, float alpha, const float *x, int incx, float *y, int incy) {
+    int64_t g = (n + kThreads * 4 - 1) / (kThreads * 4);
+    if (g > 256 * 8) g = 256 * 8;
+    const bool vec = incx == 1 && incy == 1 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+                     (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    hipStream_t s = gptc_stream_checked();
+    if (vec)
+        saxpy_vec_kernel<<<dim3(static_cast<int>(g)), dim3(kThreads), 0, s>>>(n, alpha, x, y);
+    else
+        saxpy_kernel<<<dim3(static_cast<int>(g)), dim3(kThreads), 0, s>>>(n, alpha, x, incx, y, incy);
+    hipCheck(hipGetLastError());
+}
+
+}  // namespace
+
 void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
                       const float *bias, const float *add, float *C) {
     const gptc::SplitGemm g{A, B, C, bias, add, M, N, K, lda, ldb, N, trans_a, trans_b};
@@ -240,9 +258,10 @@ void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const flo
         gptc::launch_split_gemm(g, gptc_stream_checked());
         return;
     }
-    CHECK_ERROR(add != nullptr && add != C, "gptc_linear_gemm: rocBLAS accumulates into C only.");
-    gptc_sgemm(trans_a, trans_b, M, N, K, 1.0f, A, lda, B, ldb, add != nullptr ? 1.0f : 0.0f, C, N);
-    if (bias != nullptr && M > 0 && N > 0) gptc::launch_bias_add(C, bias, M, N, gptc_stream_checked());
+    gptc_sgemm(trans_a, trans_b, M, N, K, 1.0f, A, lda, B, ldb, add == C ? 1.0f : 0.0f, C, N);
+    if (M <= 0 || N <= 0) return;
+    if (bias != nullptr) gptc::launch_bias_add(C, bias, M, N, gptc_stream_checked());
+    if (add != nullptr && add != C) launch_saxpy(static_cast<int64_t>(M) * N, 1.0f, add, 1, C, 1);
 }
 
 extern "C" void sgemm_cuda(const int TransA, const int TransB, const int M, const int N, const int K,
@@ -276,16 +295,5 @@ extern "C" void saxpy_cuda(const int n, const float alpha, const tensor_t *x, co
     if (n <= 0) return;
     check_span(x, offsetx, n, incx, "saxpy x");
     check_span(y, offsety, n, incy, "saxpy y");
-    hipStream_t s = gptc_stream_checked();
-    const float *xp = x->t + offsetx;
-    float *yp = y->t + offsety;
-    int64_t g = (static_cast<int64_t>(n) + kThreads * 4 - 1) / (kThreads * 4);
-    if (g > 256 * 8) g = 256 * 8;
-    const bool vec = incx == 1 && incy == 1 && (reinterpret_cast<uintptr_t>(xp) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(yp) & 15) == 0;
-    if (vec)
-        saxpy_vec_kernel<<<dim3(static_cast<int>(g)), dim3(kThreads), 0, s>>>(n, alpha, xp, yp);
-    else
-        saxpy_kernel<<<dim3(static_cast<int>(g)), dim3(kThreads), 0, s>>>(n, alpha, xp, incx, yp, incy);
-    hipCheck(hipGetLastError());
+    launch_saxpy(n, alpha, x->t + offsetx, incx, y->t + offsety, incy);
 }

@@ -14,7 +14,8 @@ void gptc_sgemm(int trans_a, int trans_b, int M, int N, int K, float alpha, cons
                 int ldb, float beta, float *C, int ldc);
 
 // The products of the Linear layers, row-major and without gaps in C:
-// C (M x N) = op(A) op(B) (+ bias, N values) (+ add, M x N: nullptr or C).
+// C (M x N) = op(A) op(B) (+ bias, N values) (+ add, M x N: C itself to accumulate,
+// another buffer, or nullptr).
 // Runs the kernels of gemm_split.hip where they serve, else rocBLAS.
 // Deterministic.
 void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const float *A, int lda, const float *B, int ldb,

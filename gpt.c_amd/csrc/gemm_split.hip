@@ -614,7 +614,7 @@ constexpr Tile kTiles[] = {
     {128, 64, 3, 1.20f, 0.79f, 0.79f, 1.05f},
     {64, 64, 4, 0.80f, 0.45f, 0.42f, 1.35f},
 };
-// Products of fewer multiply-adds without a bias stay with rocBLAS, whose small
+// Products of fewer multiply-adds without a bias or residual stay with rocBLAS, whose small
 // fp32 tiles start up faster (1024 x 768 x 768: 13 us against 17; 300 x 512 x 512: 8
 // against 11; from 2048 x 768 x 768, 1.2e9, on the two are level); with a bias its
 // second launch costs what that gains (Linear forward and backward of 64 rows,
@@ -729,7 +729,7 @@ bool split_gemm_serves(const SplitGemm &g) {
     constexpr int kMaxLd = 1 << 22;  // a tile's offsets (256 rows) fit 32 bits
     if (g.M <= 0 || g.N <= 0 || g.K <= 0 || (g.trans_a && g.trans_b) || g.lda >= kMaxLd || g.ldb >= kMaxLd) return false;
     const double macs = static_cast<double>(g.M) * g.N * g.K;
-    return g.bias != nullptr || macs >= kLibraryMacs;
+    return g.bias != nullptr || (g.add != nullptr && g.add != g.C) || macs >= kLibraryMacs;
 }
 
 void launch_split_gemm(const SplitGemm &g, hipStream_t stream) { run_plan(g, choose(g), stream); }

@@ -131,12 +131,13 @@ __global__ __launch_bounds__(kThreads) void layernorm_fwd4_kernel(const float *_
 
 // Workgroup blockIdx.x owns rows [r0, r1); its waves take every 4th row.
 // partial: (2, gridDim.x, C) = dW then db sums of this workgroup.
-// acc: dout += dx (the reference's semantics); otherwise dout = dx.
+// add: dout = add + dx (add = dout: the reference's accumulating form; it may alias
+// dout element by element, nothing else); nullptr: dout = dx.
 template <int K>
 __global__ __launch_bounds__(kThreads) void layernorm_bwd_kernel(
     const float *__restrict__ g, const float *__restrict__ x, const float *__restrict__ mean_in,
-    const float *__restrict__ rstd_in, const float *__restrict__ W, float *__restrict__ dout,
-    float *__restrict__ partial, int rows, int C, int rows_per_block, bool acc) {
+    const float *__restrict__ rstd_in, const float *__restrict__ W, const float *add, float *dout,
+    float *__restrict__ partial, int rows, int C, int rows_per_block) {
     extern __shared__ float red[];  // (kWaves, 2, C)
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int r0 = blockIdx.x * rows_per_block;
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd_kernel(
                 dw[k] += gv[k] * (a * xv[k] + bn);
                 dbs[k] += gv[k];
                 const float d = a * gv[k] * wv[k] + bb * xv[k] + cc;
-                dr[j] = acc ? dr[j] + d : d;
+                dr[j] = add != nullptr ? add[static_cast<int64_t>(row) * C + j] + d : d;
             }
         }
     }
@@ -204,15 +205,14 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd_kernel(
 
 // The same backward on float4 columns (C % 4 == 0, 16-byte aligned rows and
 // W): lane l holds float4 columns l, l + 64, ...  A wave takes ROWS of its
-// rows per step (r, r + 4, ...) and issues every load of them, dout's
+// rows per step (r, r + 4, ...) and issues every load of them, add's
 // included, before the first use, so a step costs one memory latency.
-// ACC: dout += dx (the reference's semantics); otherwise dout = dx and
-// dout is not read.  The dW / db sums of a column see the rows in the same
+// ACC: dout = add + dx; otherwise dout = dx.  The dW / db sums of a column see the rows in the same
 // order as in the kernel above.
 template <int K4, int ROWS, bool ACC>
 __global__ __launch_bounds__(kThreads) void layernorm_bwd4_kernel(
     const float *__restrict__ g, const float *__restrict__ x, const float *__restrict__ mean_in,
-    const float *__restrict__ rstd_in, const float *__restrict__ W, float *__restrict__ dout,
+    const float *__restrict__ rstd_in, const float *__restrict__ W, const float *add, float *dout,
     float *__restrict__ partial, int rows, int C, int rows_per_block) {
     extern __shared__ float red[];  // (kWaves, 2, C)
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd4_kernel(
             const int ri = min(row + i * kWaves, r1 - 1);
             const f32x4_t *xr = reinterpret_cast<const f32x4_t *>(x + static_cast<int64_t>(ri) * C);
             const f32x4_t *gr = reinterpret_cast<const f32x4_t *>(g + static_cast<int64_t>(ri) * C);
-            const f32x4_t *dr = reinterpret_cast<const f32x4_t *>(dout + static_cast<int64_t>(ri) * C);
+            const f32x4_t *dr = reinterpret_cast<const f32x4_t *>((ACC ? add : x) + static_cast<int64_t>(ri) * C);
 #pragma unroll
             for (int k = 0; k < K4; ++k) {
                 const int c = min(lane + k * kWave, n4 - 1);
@@ -348,11 +348,12 @@ struct FwdLaunch {
 
 template <int K>
 struct BwdLaunch {
-    static void run(const float *g, const float *x, const float *mean, const float *rstd, const float *W, float *dout,
-                    float *partial, int rows, int C, int parts, int rows_per_block, bool acc, hipStream_t s) {
+    static void run(const float *g, const float *x, const float *mean, const float *rstd, const float *W,
+                    const float *add, float *dout, float *partial, int rows, int C, int parts, int rows_per_block,
+                    hipStream_t s) {
         const size_t lds = sizeof(float) * kWaves * 2 * C;
-        layernorm_bwd_kernel<K><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, dout, partial, rows, C,
-                                                                        rows_per_block, acc);
+        layernorm_bwd_kernel<K><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, add, dout, partial, rows,
+                                                                        C, rows_per_block);
         hipCheck(hipGetLastError());
     }
 };
@@ -360,38 +361,41 @@ struct BwdLaunch {
 // Float4 columns per lane of layernorm_bwd4_kernel: 1, 2, 3, 4, 6 or 8
 // (C <= 256, 512, 768, 1024, 1536, 2048); two rows per step up to 4.
 template <int K4>
-void bwd4_launch(const float *g, const float *x, const float *mean, const float *rstd, const float *W, float *dout,
-                 float *partial, int rows, int C, int parts, int rows_per_block, bool acc, hipStream_t s) {
+void bwd4_launch(const float *g, const float *x, const float *mean, const float *rstd, const float *W,
+                 const float *add, float *dout, float *partial, int rows, int C, int parts, int rows_per_block,
+                 hipStream_t s) {
     constexpr int R = K4 <= 4 ? 2 : 1;
     const size_t lds = sizeof(float) * kWaves * 2 * C;
-    if (acc)
-        layernorm_bwd4_kernel<K4, R, true><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, dout,
+    if (add != nullptr)
+        layernorm_bwd4_kernel<K4, R, true><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, add, dout,
                                                                                    partial, rows, C, rows_per_block);
     else
-        layernorm_bwd4_kernel<K4, R, false><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, dout,
+        layernorm_bwd4_kernel<K4, R, false><<<dim3(parts), dim3(kThreads), lds, s>>>(g, x, mean, rstd, W, add, dout,
                                                                                     partial, rows, C, rows_per_block);
     hipCheck(hipGetLastError());
 }
 
-// dout (+)= dx, dW += ..., db += ... of rows x C (1 <= C <= kMaxCols).
+// dout = (add +) dx, dW += ..., db += ... of rows x C (1 <= C <= kMaxCols).
 void layer_norm_backward(const float *g, const float *x, const float *mean, const float *rstd, const float *W,
-                         float *dout, float *dW, float *db, int rows, int C, bool acc, hipStream_t s) {
+                         const float *add, float *dout, float *dW, float *db, int rows, int C, hipStream_t s) {
     // About 4 rows per wave: 512 workgroups (two per CU) at GPT-2's 8192 rows.
     int parts = (rows + 15) / 16;
     if (parts > 1024) parts = 1024;
     const int rows_per_block = (rows + parts - 1) / parts;
     parts = (rows + rows_per_block - 1) / rows_per_block;
     float *partial = static_cast<float *>(alloc_cuda(sizeof(float) * 2 * static_cast<size_t>(parts) * C));
-    if (C % 4 == 0 && aligned16(g) && aligned16(x) && aligned16(W) && aligned16(dout)) {
+    if (C % 4 == 0 && aligned16(g) && aligned16(x) && aligned16(W) && aligned16(dout) && aligned16(add)) {
         const int k4 = (C / 4 + kWave - 1) / kWave;
         auto f = k4 <= 1 ? bwd4_launch<1> : k4 <= 2 ? bwd4_launch<2> : k4 <= 3 ? bwd4_launch<3>
                : k4 <= 4 ? bwd4_launch<4> : k4 <= 6 ? bwd4_launch<6> : bwd4_launch<8>;
-        f(g, x, mean, rstd, W, dout, partial, rows, C, parts, rows_per_block, acc, s);
+        f(g, x, mean, rstd, W, add, dout, partial, rows, C, parts, rows_per_block, s);
     } else {
-        by_cols<BwdLaunch>(C, g, x, mean, rstd, W, dout, partial, rows, C, parts, rows_per_block, acc, s);
+        by_cols<BwdLaunch>(C, g, x, mean, rstd, W, add, dout, partial, rows, C, parts, rows_per_block, s);
     }
-    launch_add_column_partials(partial, dW, parts, C, s);
-    if (db != nullptr) launch_add_column_partials(partial + static_cast<size_t>(parts) * C, db, parts, C, s);
+    // Both sums in one launch; one after the other if a caller passes one buffer for both.
+    const bool same = db == dW;
+    launch_add_column_partials(partial, dW, parts, C, s, same ? nullptr : db);
+    if (same) launch_add_column_partials(partial + static_cast<size_t>(parts) * C, db, parts, C, s);
     free_cuda(partial);
 }
 
@@ -443,7 +447,7 @@ extern "C" void layer_norm_forward_cuda_kernel(const tensor_t *W, const tensor_t
 namespace {
 
 void layer_norm_backward_checked(const tensor_t *global_grad, const tensor_t **cache, const tensor_t *W, tensor_t *dW,
-                                 tensor_t *db, tensor_t *dout, bool acc) {
+                                 tensor_t *db, const tensor_t *add, tensor_t *dout) {
     check_gpu(global_grad, "global_grad");
     REQUIRE_ARG(cache);
     check_gpu(cache[0], "cache[0] (mean)");
@@ -462,19 +466,30 @@ void layer_norm_backward_checked(const tensor_t *global_grad, const tensor_t **c
         check_gpu(db, "db");
         CHECK_ERROR(db->length != C, "Expected db to hold %d elements, but got %d.", C, db->length);
     }
+    if (add != NULL) {
+        check_gpu(add, "add");
+        CHECK_ERROR(add->length != dout->length, "Expected add to match dout's %d elements, but got %d.", dout->length,
+                    add->length);
+    }
     if (rows == 0) return;
-    layer_norm_backward(global_grad->t, cache[2]->t, cache[0]->t, cache[1]->t, W->t, dout->t, dW->t,
-                        db != NULL ? db->t : nullptr, rows, C, acc, gptc_stream_checked());
+    layer_norm_backward(global_grad->t, cache[2]->t, cache[0]->t, cache[1]->t, W->t, add != NULL ? add->t : nullptr,
+                        dout->t, dW->t, db != NULL ? db->t : nullptr, rows, C, gptc_stream_checked());
 }
 
 }  // namespace
 
 extern "C" void layer_norm_backward_cuda_kernel(const tensor_t *global_grad, const tensor_t **cache,
                                                 const tensor_t *W, tensor_t *dW, tensor_t *db, tensor_t *dout) {
-    layer_norm_backward_checked(global_grad, cache, W, dW, db, dout, true);
+    layer_norm_backward_checked(global_grad, cache, W, dW, db, dout, dout);
 }
 
 extern "C" void gptc_layer_norm_backward_set(const tensor_t *global_grad, const tensor_t **cache, const tensor_t *W,
                                              tensor_t *dW, tensor_t *db, tensor_t *dout) {
-    layer_norm_backward_checked(global_grad, cache, W, dW, db, dout, false);
+    layer_norm_backward_checked(global_grad, cache, W, dW, db, NULL, dout);
+}
+
+extern "C" void gptc_layer_norm_backward_add(const tensor_t *global_grad, const tensor_t **cache, const tensor_t *W,
+                                             tensor_t *dW, tensor_t *db, const tensor_t *add, tensor_t *dout) {
+    REQUIRE_ARG(add);
+    layer_norm_backward_checked(global_grad, cache, W, dW, db, add, dout);
 }

@@ -61,12 +61,17 @@ __global__ __launch_bounds__(kThreads) void colsum_partial_kernel(const float *_
 
 constexpr int kPartialWaves = 8;
 
-// out[c] += sum over p < parts of partial[p, c].  A workgroup owns 64
+// out[c] += sum over p < parts of partial[p, c]; blockIdx.y = 1: the same of the
+// parts that follow, into out2.  A workgroup owns 64
 // columns; wave w adds rows p = w, w + 8, ... and the 8 wave sums are then
 // added in wave order, so the result does not depend on scheduling.
 __global__ __launch_bounds__(kPartialWaves * kWave) void add_column_partials_kernel(const float *__restrict__ partial,
-                                                                                  float *__restrict__ out, int parts,
-                                                                                  int cols) {
+                                                                                  float *out, int parts, int cols,
+                                                                                  float *out2) {
+    if (blockIdx.y == 1) {
+        partial += static_cast<int64_t>(parts) * cols;
+        out = out2;
+    }
     __shared__ float red[kPartialWaves][kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int c = blockIdx.x * kWave + lane;
@@ -118,11 +123,16 @@ __global__ __launch_bounds__(kThreads) void colsum_partial4_kernel(const float *
 
 constexpr int kSlices = 32;  // part slices per workgroup of add_column_partials4_kernel
 
-// out[c] += sum over p < parts of partial[p, c]: thread (slice sl, float4
+// out[c] += sum over p < parts of partial[p, c] (and the next parts into out2, as
+// above): thread (slice sl, float4
 // column c4) adds parts sl, sl + 32, ... into four alternating sums (added in
 // order), and the 32 slice sums are then added in slice order.
 __global__ __launch_bounds__(kThreads) void add_column_partials4_kernel(const float *__restrict__ partial,
-                                                                       float *__restrict__ out, int parts, int cols) {
+                                                                       float *out, int parts, int cols, float *out2) {
+    if (blockIdx.y == 1) {
+        partial += static_cast<int64_t>(parts) * cols;
+        out = out2;
+    }
     constexpr int kGroups = kThreads / kSlices;  // float4 columns per workgroup
     __shared__ f32x4_t red[kSlices][kGroups];
     const int cl = threadIdx.x % kGroups, sl = threadIdx.x / kGroups;
@@ -193,17 +203,18 @@ void launch_column_sum_add(const float *g, float *out, int rows, int cols, hipSt
     free_cuda(partial);
 }
 
-void launch_add_column_partials(const float *partial, float *out, int parts, int cols, hipStream_t s) {
+void launch_add_column_partials(const float *partial, float *out, int parts, int cols, hipStream_t s, float *out2) {
     if (parts <= 0 || cols <= 0) return;
-    if (cols % 4 == 0 && aligned16p(partial) && aligned16p(out)) {
+    const int sums = out2 != nullptr ? 2 : 1;
+    if (cols % 4 == 0 && aligned16p(partial) && aligned16p(out) && aligned16p(out2)) {
         const int groups = kThreads / kSlices;
-        add_column_partials4_kernel<<<dim3((cols / 4 + groups - 1) / groups), dim3(kThreads), 0, s>>>(partial, out,
-                                                                                                     parts, cols);
+        add_column_partials4_kernel<<<dim3((cols / 4 + groups - 1) / groups, sums), dim3(kThreads), 0, s>>>(
+            partial, out, parts, cols, out2);
         hipCheck(hipGetLastError());
         return;
     }
-    add_column_partials_kernel<<<dim3((cols + kWave - 1) / kWave), dim3(kPartialWaves * kWave), 0, s>>>(partial, out,
-                                                                                                     parts, cols);
+    add_column_partials_kernel<<<dim3((cols + kWave - 1) / kWave, sums), dim3(kPartialWaves * kWave), 0, s>>>(
+        partial, out, parts, cols, out2);
     hipCheck(hipGetLastError());
 }
 
@@ -211,8 +222,11 @@ void launch_add_column_partials(const float *partial, float *out, int parts, int
 
 using namespace gptc;
 
-extern "C" void linear_forward_cuda_kernel(const tensor_t *W, const tensor_t *b, const tensor_t *input,
-                                           tensor_t *output) {
+namespace {
+
+// output = input W^T (+ b) (+ add)
+void linear_forward(const tensor_t *W, const tensor_t *b, const tensor_t *input, const tensor_t *add,
+                    tensor_t *output) {
     check_gpu(W, "W");
     check_gpu(input, "input");
     check_gpu(output, "output");
@@ -227,8 +241,26 @@ extern "C" void linear_forward_cuda_kernel(const tensor_t *W, const tensor_t *b,
         check_gpu(b, "b");
         CHECK_ERROR(b->length != out_f, "Expected b to hold %d elements, but got %d.", out_f, b->length);
     }
-    gptc_linear_gemm(false, true, rows, out_f, in_f, input->t, in_f, W->t, in_f, b != NULL ? b->t : nullptr, nullptr,
-                     output->t);
+    if (add != NULL) {
+        check_gpu(add, "add");
+        CHECK_ERROR(add->length != output->length, "Expected add to match output's %d elements, but got %d.",
+                    output->length, add->length);
+    }
+    gptc_linear_gemm(false, true, rows, out_f, in_f, input->t, in_f, W->t, in_f, b != NULL ? b->t : nullptr,
+                     add != NULL ? add->t : nullptr, output->t);
+}
+
+}  // namespace
+
+extern "C" void linear_forward_cuda_kernel(const tensor_t *W, const tensor_t *b, const tensor_t *input,
+                                           tensor_t *output) {
+    linear_forward(W, b, input, NULL, output);
+}
+
+extern "C" void gptc_linear_forward_add_cuda(const tensor_t *W, const tensor_t *b, const tensor_t *input,
+                                             const tensor_t *add, tensor_t *output) {
+    REQUIRE_ARG(add);
+    linear_forward(W, b, input, add, output);
 }
 
 extern "C" void linear_backward_cuda_kernel(const tensor_t *global_grad, const tensor_t *cache, const tensor_t *W,

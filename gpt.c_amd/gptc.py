@@ -189,6 +189,13 @@ SIGNATURES = {
     "layer_norm_backward_cuda_kernel": (None, [TensorP, ctypes.POINTER(TensorP), TensorP, TensorP, TensorP,
                                                TensorP]),
     "gptc_layer_norm_backward_set": (None, [TensorP, ctypes.POINTER(TensorP), TensorP, TensorP, TensorP, TensorP]),
+    "gptc_layer_norm_backward_add": (None, [TensorP, ctypes.POINTER(TensorP), TensorP, TensorP, TensorP, TensorP,
+                                            TensorP]),
+    "gptc_linear_forward_add_cuda": (None, [TensorP, TensorP, TensorP, TensorP, TensorP]),
+    "gptc_linear_forward_residual": (TensorP, [_vp, TensorP, TensorP]),
+    "gptc_layer_norm_backward_residual": (TensorP, [_vp, TensorP, TensorP]),
+    "gptc_mlp_forward_residual": (TensorP, [_vp, TensorP, TensorP]),
+    "gptc_self_attention_forward_residual": (TensorP, [_vp, TensorP, TensorP]),
     "gelu_forward_cuda_kernel": (None, [TensorP, TensorP]),
     "gelu_backward_cuda_kernel": (None, [TensorP, TensorP, TensorP]),
     "softmax_forward_cuda_kernel": (None, [TensorP, TensorP]),

@@ -94,6 +94,10 @@ mlp_t *MLP(const int in_features, int expansion_factor, const int use_bias);
 self_attention_t *SelfAttention(const int n_embd, const int n_heads, const int block_size, const int use_bias);
 block_t *Block(const int n_embd, const int n_heads, const int block_size, const int use_bias);
 
+/* forward(x) + residual (the residual is read, not consumed): Block's two adds. */
+tensor_t *gptc_mlp_forward_residual(mlp_t *mlp, tensor_t *x, const tensor_t *residual);
+tensor_t *gptc_self_attention_forward_residual(self_attention_t *sa, tensor_t *x, const tensor_t *residual);
+
 #ifdef __cplusplus
 }
 #endif

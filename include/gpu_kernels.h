@@ -150,6 +150,19 @@ void gptc_layer_norm_backward_set(const tensor_t *global_grad, const tensor_t **
                                   tensor_t *dW, tensor_t *db, tensor_t *dout);
 
 /*
+ * gptc_layer_norm_backward_add(global_grad, cache, W, dW, db, add, dout)
+ *   The same with dout = add + dx: the residual's gradient joined in the pass
+ *   that writes dx (gpt.c's Block adds it with a saxpy, src/block.c:108,124).
+ * gptc_linear_forward_add_cuda(W, b, input, add, output)
+ *   linear_forward_cuda_kernel with output = input W^T + b + add: the residual
+ *   likewise (src/block.c:68,82).
+ */
+void gptc_layer_norm_backward_add(const tensor_t *global_grad, const tensor_t **cache, const tensor_t *W,
+                                  tensor_t *dW, tensor_t *db, const tensor_t *add, tensor_t *dout);
+void gptc_linear_forward_add_cuda(const tensor_t *W, const tensor_t *b, const tensor_t *input, const tensor_t *add,
+                                  tensor_t *output);
+
+/*
  * ---- the rest of gpt.c's GPU back end (the other layers of the model) ----
  * Same names, arguments and meaning as the CUDA entry points they replace;
  * the semantics are those of gpt.c's CPU kernels (kernels/src/cpu/), which

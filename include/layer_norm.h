@@ -37,6 +37,9 @@ typedef struct layer_norm {
 
 layer_norm_t *LayerNorm(int in_features, const float eps, const int use_bias);
 
+/* backward(global_grad) + residual (the residual is read, not consumed). */
+tensor_t *gptc_layer_norm_backward_residual(layer_norm_t *norm, tensor_t *global_grad, const tensor_t *residual);
+
 #ifdef __cplusplus
 }
 #endif

@@ -47,6 +47,9 @@ linear_t *Linear(const int in_features, const int out_features, const int use_bi
 tensor_t *gptc_linear_forward_nobias(linear_t *linear, tensor_t *x);
 tensor_t *gptc_linear_backward_nodb(linear_t *linear, tensor_t *global_grad);
 
+/* forward(x) + residual (the residual is read, not consumed). */
+tensor_t *gptc_linear_forward_residual(linear_t *linear, tensor_t *x, const tensor_t *residual);
+
 #ifdef __cplusplus
 }
 #endif
