@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include <cstdint>
+#include "wave_reduce.hpp"
 
 namespace gptc {
 
@@ -165,24 +166,5 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 
 // Value held by the lane 32 positions away (the other half of the wave).
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
-
-// Max and sum over the four lanes l % 16 + {0, 16, 32, 48} (one query of a
-// 16 x 16 accumulator), every lane receiving the result.  gfx950's
-// v_permlane32_swap / v_permlane16_swap exchange lane halves / 16-lane rows
-// in the VALU: with both operands equal to x, the two results hold x at the
-// lane and at its partner (l ^ 32, then l ^ 16), in some order.
-__device__ __forceinline__ float max4_rows(float x) {
-    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-__device__ __forceinline__ float sum4_rows(float x) {
-    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 }  // namespace gptc

@@ -37,11 +37,7 @@ constexpr int kDecWaves = kDecThreads / 64;
 
 __device__ __forceinline__ float block_reduce(float v, float *red, bool is_max) {
     // Wave reduction, then the wave results through LDS (a fixed order).
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float o = __shfl_xor(v, off, 64);
-        v = is_max ? fmaxf(v, o) : v + o;
-    }
+    v = is_max ? wave_max(v) : wave_sum(v);
     const int w = threadIdx.x >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[w] = v;
@@ -242,22 +238,18 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const DecParams 
                 acc = fmaf(q4[3], k4[3], acc);
             }
         }
-        acc += __shfl_xor(acc, 1, 64);
-        acc += __shfl_xor(acc, 2, 64);
+        acc += dpp_of<kDppXor1>(acc);  // the key's four threads
+        acc += dpp_of<kDppXor2>(acc);
         if (kk < n) t = acc * a.scale_log2;
     }
-    float m = t;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    float m = wave_max(t);
     if (lane == 0) red[w] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const float p = kk < n ? fast_exp2(t - m) : 0.0f;
     if (qq == 0) p_s[kk] = p;
     // The sum of p over the chunk (each key counted by its qq == 0 thread).
-    float l = qq == 0 ? p : 0.0f;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
+    const float l = wave_sum(qq == 0 ? p : 0.0f);
     __syncthreads();  // p_s complete; red[] read by everyone
     if (lane == 0) red[w] = l;
 
@@ -364,15 +356,13 @@ __device__ __forceinline__ void decode_head_rounds(const DecParams &a, int pos, 
         acc = fmaf(q4[1], k4[r][1], acc);
         acc = fmaf(q4[2], k4[r][2], acc);
         acc = fmaf(q4[3], k4[r][3], acc);
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) acc += __shfl_xor(acc, off, 64);
+        acc = row16_sum(acc);
         const int j = 64 * r + 4 * w + (lane >> 4);
         t[r] = j < n ? acc * a.scale_log2 : -INFINITY;
         mx = fmaxf(mx, t[r]);
     }
     // The four row groups of the wave, then the 16 waves.
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max4_rows(mx);
     if (lane == 0) m_red[w] = mx;
     __syncthreads();
     float m = m_red[0];
@@ -387,12 +377,9 @@ __device__ __forceinline__ void decode_head_rounds(const DecParams &a, int pos, 
         l += p;
         o += p * v4[r];
     }
+    l = sum4_rows(l);
 #pragma unroll
-    for (int off = 16; off < 64; off <<= 1) {
-        l += __shfl_xor(l, off, 64);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], off, 64);
-    }
+    for (int e = 0; e < 4; ++e) o[e] = sum4_rows(o[e]);
     if (lane < 16) *reinterpret_cast<f32x4 *>(&o_red[w][4 * lane]) = o;
     if (lane == 0) l_red[w] = l;
     __syncthreads();

@@ -31,18 +31,6 @@ namespace {
 
 constexpr int kGenWaves = 4;  // queries (or keys) per workgroup
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // Keys (or queries) per staged chunk for head size D: the largest of 64, 32,
 // 16 and 8 with which the two tiles of KC x (D + 1) and KC x D floats, the
 // waves' rows and weights (and 2 KB of static LDS) stay within 150 KB.
