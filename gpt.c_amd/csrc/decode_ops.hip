@@ -38,7 +38,7 @@ struct RowsArgs {
 // The 4 waves of a workgroup own `kOuts` groups of kPer output features;
 // for each group, the kSplit = 4 / kOuts waves on it take equal slices of the
 // in_f inputs (so a narrow output still puts work on every CU), and the
-// slices' sums meet in LDS.  acc[p][r] = W[o_p, :] . xn[r, :] for r < rows,
+// slices' sums meet in LDS.  acc[p][r] = W[o_p, :] . xn[r, :] for r < kRows,
 // where xn = x, or with kLN the LayerNorm of each x row (mean and rstd
 // computed by the workgroup: the decode step's rows are at most 8 of a few
 // thousand features).  kPer > 1 (wide outputs): a wave reads its normalised
@@ -49,7 +49,9 @@ struct RowsArgs {
 // wave's first kIt 16-byte weight vectors, the LayerNorm weights, the bias
 // and residual of the output this thread finishes) is requested before
 // them, and the sums keep the order of a plain loop over the inputs.
-template <bool kVec, bool kLN, int kOuts, int kPer>
+// kRows: a compile-time bound on the rows, so that their chains interleave
+// without branches; rows past a.rows repeat the last and are not written.
+template <bool kVec, bool kLN, int kOuts, int kPer, int kRows>
 __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a) {
     constexpr int kSplit = kWaves / kOuts;
     // 16-byte steps per lane loaded up front (in_f <= 1024 kSplit).  Wide
@@ -57,8 +59,8 @@ __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a)
     // instead: their registers buy occupancy there (34 against 40 us).
     constexpr int kIt = kPer == 1 ? 4 : 0;
     constexpr int kItN = kIt > 0 ? kIt : 1;
-    __shared__ float part[kWaves * kPer][kMaxRows];
-    __shared__ float stat[2][kMaxRows];
+    __shared__ float part[kWaves * kPer][kRows];
+    __shared__ float stat[2][kRows];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int in_f = a.in_f, rows = a.rows;
     const int grp = w / kSplit, slice = w % kSplit;
@@ -138,29 +140,28 @@ __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a)
         }
         __syncthreads();
     }
-    float acc[kPer][kMaxRows];
+    float acc[kPer][kRows];
 #pragma unroll
     for (int p = 0; p < kPer; ++p)
 #pragma unroll
-        for (int r = 0; r < kMaxRows; ++r) acc[p][r] = 0.0f;
+        for (int r = 0; r < kRows; ++r) acc[p][r] = 0.0f;
     if (o0 < a.out_f) {
         if (kVec) {  // in_f % (4 kSplit) == 0: slices are whole 16-byte vectors
             auto step = [&](int j, const f32x4_t(&w4)[kPer], const f32x4_t &lw4, const f32x4_t &lb4) {
 #pragma unroll
-                for (int r = 0; r < kMaxRows; ++r) {
-                    if (r < rows) {
-                        f32x4_t xv = reinterpret_cast<const f32x4_t *>(a.x + static_cast<int64_t>(r) * in_f)[j];
-                        if (kLN) {
+                for (int r = 0; r < kRows; ++r) {
+                    const int rc = min(r, rows - 1);
+                    f32x4_t xv = reinterpret_cast<const f32x4_t *>(a.x + static_cast<int64_t>(rc) * in_f)[j];
+                    if (kLN) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) xv[e] = (xv[e] - stat[0][r]) * stat[1][r] * lw4[e] + lb4[e];
-                        }
+                        for (int e = 0; e < 4; ++e) xv[e] = (xv[e] - stat[0][rc]) * stat[1][rc] * lw4[e] + lb4[e];
+                    }
 #pragma unroll
-                        for (int p = 0; p < kPer; ++p) {
-                            acc[p][r] = fmaf(w4[p][0], xv[0], acc[p][r]);
-                            acc[p][r] = fmaf(w4[p][1], xv[1], acc[p][r]);
-                            acc[p][r] = fmaf(w4[p][2], xv[2], acc[p][r]);
-                            acc[p][r] = fmaf(w4[p][3], xv[3], acc[p][r]);
-                        }
+                    for (int p = 0; p < kPer; ++p) {
+                        acc[p][r] = fmaf(w4[p][0], xv[0], acc[p][r]);
+                        acc[p][r] = fmaf(w4[p][1], xv[1], acc[p][r]);
+                        acc[p][r] = fmaf(w4[p][2], xv[2], acc[p][r]);
+                        acc[p][r] = fmaf(w4[p][3], xv[3], acc[p][r]);
                     }
                 }
             };
@@ -185,16 +186,15 @@ __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a)
         } else {
             for (int j = j0 + lane; j < j1; j += kWave) {
 #pragma unroll
-                for (int r = 0; r < kMaxRows; ++r) {
-                    if (r < rows) {
-                        float xv = a.x[static_cast<int64_t>(r) * in_f + j];
-                        if (kLN)
-                            xv = (xv - stat[0][r]) * stat[1][r] * a.ln_w[j] + (a.ln_b != nullptr ? a.ln_b[j] : 0.0f);
+                for (int r = 0; r < kRows; ++r) {
+                    const int rc = min(r, rows - 1);
+                    float xv = a.x[static_cast<int64_t>(rc) * in_f + j];
+                    if (kLN)
+                        xv = (xv - stat[0][rc]) * stat[1][rc] * a.ln_w[j] + (a.ln_b != nullptr ? a.ln_b[j] : 0.0f);
 #pragma unroll
-                        for (int p = 0; p < kPer; ++p)
-                            if (o0 + p < a.out_f)
-                                acc[p][r] = fmaf(a.W[static_cast<int64_t>(o0 + p) * in_f + j], xv, acc[p][r]);
-                    }
+                    for (int p = 0; p < kPer; ++p)
+                        if (o0 + p < a.out_f)
+                            acc[p][r] = fmaf(a.W[static_cast<int64_t>(o0 + p) * in_f + j], xv, acc[p][r]);
                 }
             }
         }
@@ -202,11 +202,10 @@ __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a)
 #pragma unroll
     for (int p = 0; p < kPer; ++p)
 #pragma unroll
-        for (int r = 0; r < kMaxRows; ++r)
-            if (r < rows) {
-                const float v = wave_sum(acc[p][r]);
-                if (lane == 0) part[(grp * kPer + p) * kSplit + slice][r] = v;
-            }
+        for (int r = 0; r < kRows; ++r) {
+            const float v = wave_sum(acc[p][r]);
+            if (lane == 0) part[(grp * kPer + p) * kSplit + slice][r] = v;
+        }
     __syncthreads();
     // One thread per (output, row) adds the slices in order and finishes.
     for (int t = threadIdx.x; t < n_fin; t += kThreads) {
@@ -225,13 +224,175 @@ __global__ __launch_bounds__(kThreads) void linear_rows_kernel(const RowsArgs a)
     }
 }
 
+// LayerNorm and product for rows of at most 1024 whole 16-byte vectors' floats
+// (kHeldVecs per lane), every load requested before the first use:
+//   ln_row_held   one row: a wave per output feature forms the statistics from
+//                 the registers its dot product then takes, and writes its
+//                 output without LDS or a barrier.  That each wave forms them
+//                 again costs less than the barrier and the second read of x.
+//   ln_rows_held  2 .. 8 rows: the waves of a workgroup normalise the rows into
+//                 LDS, and each then dots its weight row with them.
+// us a token of 12 layers, C = 768, with linear_rows_kernel and a run-time row count
+// everywhere -> these -> and compile-time row counts in the remaining launches:
+//   GPT-2 small (50257 outputs, 512 keys), 1 row 357 -> 343 -> 331
+//   1000 outputs, 2 rows 311 -> 283 -> 267   4 rows 359 -> 321 -> 290
+//                 6 rows 416 -> 386 -> 360   8 rows 464 -> 418 -> 370
+constexpr int kHeldVecs = 4;
+constexpr int kHeldOuts = 8192;  // several rows: narrower outputs than this
+
+__device__ __forceinline__ void finish_row(const RowsArgs &a, int o, int r, float y, float bias, float res) {
+    if (a.b != nullptr) y += bias;
+    if (a.act == 1) y = gelu_tanh(y);
+    if (a.res != nullptr) y += res;
+    a.y[static_cast<int64_t>(r) * a.out_f + o] = y;
+}
+
+__device__ __forceinline__ f32x4_t load4_or_zero(const float *p, int j, bool ok) {
+    return ok ? reinterpret_cast<const f32x4_t *>(p)[j] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+}
+
+struct RowStat {
+    float mean, rstd;
+};
+
+// As layer_norm_forward_cuda_kernel forms them: mean and E[x^2] - mean^2.
+__device__ __forceinline__ RowStat stat_held(const f32x4_t (&x)[kHeldVecs], const RowsArgs &a) {
+    float s = 0.0f, ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHeldVecs; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s += x[i][e];
+            ss += x[i][e] * x[i][e];
+        }
+    s = wave_sum(s);
+    ss = wave_sum(ss);
+    const float scale = 1.0f / a.in_f;
+    const float mean = s * scale;
+    return {mean, 1.0f / sqrtf(ss * scale - mean * mean + a.eps)};
+}
+
+__global__ __launch_bounds__(kThreads) void ln_row_held_kernel(const RowsArgs a) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int o = blockIdx.x * kWaves + w;
+    if (o >= a.out_f) return;
+    const int n4 = a.in_f / 4;
+    f32x4_t wv[kHeldVecs], lw[kHeldVecs], lb[kHeldVecs], x[kHeldVecs];
+#pragma unroll
+    for (int i = 0; i < kHeldVecs; ++i) {
+        const int j = lane + i * kWave;
+        const bool ok = j < n4;
+        wv[i] = load4_or_zero(a.W + static_cast<int64_t>(o) * a.in_f, j, ok);
+        x[i] = load4_or_zero(a.x, j, ok);
+        lw[i] = load4_or_zero(a.ln_w, j, ok);
+        lb[i] = load4_or_zero(a.ln_b, j, ok && a.ln_b != nullptr);
+    }
+    float bias = 0.0f, res = 0.0f;
+    if (lane == 0) {
+        if (a.b != nullptr) bias = a.b[o];
+        if (a.res != nullptr) res = a.res[o];
+    }
+    const RowStat st = stat_held(x, a);
+    float acc = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHeldVecs; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (lane + i * kWave < n4)  // past the row nothing, also where mean or rstd is not finite
+                acc = fmaf(wv[i][e], (x[i][e] - st.mean) * st.rstd * lw[i][e] + lb[i][e], acc);
+    acc = wave_sum(acc);
+    if (lane == 0) finish_row(a, o, 0, acc, bias, res);
+}
+
+// kRows: rows held, a compile-time count so that their chains interleave;
+// rows past a.rows repeat the last and are not written.
+template <int kRows>
+__global__ __launch_bounds__(kThreads) void ln_rows_held_kernel(const RowsArgs a) {
+    __shared__ f32x4_t xn[kRows][kHeldVecs * kWave];
+    constexpr int kMine = (kRows + kWaves - 1) / kWaves;  // rows a wave normalises
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int o = blockIdx.x * kWaves + w, oc = min(o, a.out_f - 1);
+    f32x4_t wv[kHeldVecs], lw[kHeldVecs], lb[kHeldVecs], x[kMine][kHeldVecs];
+#pragma unroll
+    for (int i = 0; i < kHeldVecs; ++i) {
+        const int j = lane + i * kWave;
+        const bool ok = j < a.in_f / 4;
+#pragma unroll
+        for (int m = 0; m < kMine; ++m)
+            x[m][i] = load4_or_zero(a.x + static_cast<int64_t>(min(w + m * kWaves, a.rows - 1)) * a.in_f, j, ok);
+        lw[i] = load4_or_zero(a.ln_w, j, ok);
+        lb[i] = load4_or_zero(a.ln_b, j, ok && a.ln_b != nullptr);
+        wv[i] = load4_or_zero(a.W + static_cast<int64_t>(oc) * a.in_f, j, ok);
+    }
+    // Lane r finishes row r.
+    const float bias = a.b != nullptr ? a.b[oc] : 0.0f;
+    const float res = a.res != nullptr && lane < a.rows ? a.res[static_cast<int64_t>(lane) * a.out_f + oc] : 0.0f;
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+        if (w + m * kWaves >= kRows) break;
+        const RowStat st = stat_held(x[m], a);
+#pragma unroll
+        for (int i = 0; i < kHeldVecs; ++i) {
+            f32x4_t v = x[m][i];
+            if (lane + i * kWave < a.in_f / 4)  // zero past the row, also where mean or rstd is not finite
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (v[e] - st.mean) * st.rstd * lw[i][e] + lb[i][e];
+            xn[w + m * kWaves][lane + i * kWave] = v;
+        }
+    }
+    __syncthreads();
+    float acc[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHeldVecs; ++i)
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            const f32x4_t v = xn[r][lane + i * kWave];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r] = fmaf(wv[i][e], v[e], acc[r]);
+        }
+    float y = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        const float v = wave_sum(acc[r]);
+        if (lane == r) y = v;
+    }
+    if (lane < a.rows && o < a.out_f) finish_row(a, o, lane, y, bias, res);
+}
+
+template <int kRows>
+void launch_ln_rows_held(const RowsArgs &a, hipStream_t s) {
+    ln_rows_held_kernel<kRows><<<dim3((a.out_f + kWaves - 1) / kWaves), dim3(kThreads), 0, s>>>(a);
+    hipCheck(hipGetLastError());
+}
+
+void run_ln_held(const RowsArgs &a, hipStream_t s) {
+    if (a.rows == 1) {
+        ln_row_held_kernel<<<dim3((a.out_f + kWaves - 1) / kWaves), dim3(kThreads), 0, s>>>(a);
+        hipCheck(hipGetLastError());
+    } else if (a.rows == 2) {
+        launch_ln_rows_held<2>(a, s);
+    } else if (a.rows <= 4) {
+        launch_ln_rows_held<4>(a, s);
+    } else {
+        launch_ln_rows_held<8>(a, s);
+    }
+}
+
 template <bool kLN, int kOuts, int kPer>
 void launch_rows(const RowsArgs &a, bool vec, hipStream_t s) {
     const dim3 grid((a.out_f + kOuts * kPer - 1) / (kOuts * kPer));
-    if (vec)
-        linear_rows_kernel<true, kLN, kOuts, kPer><<<grid, dim3(kThreads), 0, s>>>(a);
+    if (!vec)
+        linear_rows_kernel<false, kLN, kOuts, kPer, kMaxRows><<<grid, dim3(kThreads), 0, s>>>(a);
+    else if (a.rows == 1)
+        linear_rows_kernel<true, kLN, kOuts, kPer, 1><<<grid, dim3(kThreads), 0, s>>>(a);
+    else if (a.rows == 2)
+        linear_rows_kernel<true, kLN, kOuts, kPer, 2><<<grid, dim3(kThreads), 0, s>>>(a);
+    else if (a.rows <= 4)
+        linear_rows_kernel<true, kLN, kOuts, kPer, 4><<<grid, dim3(kThreads), 0, s>>>(a);
     else
-        linear_rows_kernel<false, kLN, kOuts, kPer><<<grid, dim3(kThreads), 0, s>>>(a);
+        linear_rows_kernel<true, kLN, kOuts, kPer, kMaxRows><<<grid, dim3(kThreads), 0, s>>>(a);
     hipCheck(hipGetLastError());
 }
 
@@ -243,6 +404,18 @@ void run_rows(const RowsArgs &a, hipStream_t s) {
     const int split = kind == 0 ? 4 : 1;
     const bool vec = (a.in_f % (4 * split)) == 0 && aligned16(a.W) && aligned16(a.x) &&
                      (a.ln_w == nullptr || (aligned16(a.ln_w) && aligned16(a.ln_b)));
+    // Rows that a wave holds (in_f <= 1024, whole vectors).  With several rows only
+    // up to 8192 outputs: past that the four outputs for which a wave of
+    // linear_rows_kernel reads an x vector once pay.  us a token, held against
+    // linear_rows_kernel, 8 rows: 12 layers whose MLP is 4096 wide 458 / 496, one layer
+    // and 12000 outputs 41.4 / 40.4, and 50257 outputs 73 / 63.  One row: the same
+    // 357 / 373, 28.1 / 28.6, 42.8 / 44.1; below 1024 outputs (12 layers of C = 128)
+    // 191 / 206, with 8 rows 234 / 264.
+    if (a.ln_w != nullptr && (a.rows == 1 || a.out_f < kHeldOuts) && a.in_f % 4 == 0 && a.in_f <= 4 * kHeldVecs * kWave &&
+        aligned16(a.W) && aligned16(a.x) && aligned16(a.ln_w) && aligned16(a.ln_b)) {
+        run_ln_held(a, s);
+        return;
+    }
     if (a.ln_w != nullptr) {
         if (kind == 0) launch_rows<true, 1, 1>(a, vec, s);
         else if (kind == 1) launch_rows<true, 4, 1>(a, vec, s);
