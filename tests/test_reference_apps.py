@@ -82,6 +82,7 @@ def test_cpu_device_is_refused_loudly(tmp_path):
 
 @pytest.mark.gpu
 def test_train_gpt_matches_oracle(oracle, tmp_path):
+    need(TRAIN)
     block, V, L, H, C = 64, 211, 2, 4, 96
     B, T, vB, vT = 4, 48, 2, 64
     lr, wd, eps = 1e-3, 0.1, 1e-4  # eps: see the AdamW note in test_gpt2_gpu.py
@@ -150,6 +151,7 @@ def xorshift_coins(seed, n):
 
 @pytest.mark.gpu
 def test_infer_gpt_samples_match_oracle(oracle, tmp_path):
+    need(INFER)
     block, V, L, H, C = 32, 50257, 1, 2, 64
     prompt, max_tokens, seed, temp = [11, 500, 7, 42000, 3], 40, 1234, 0.8
     params = init_params(V, block, L, C, 5, 0.3)
