@@ -3,11 +3,13 @@ blocks, slabs and tiles, against the oracle at the tolerance of
 tests/test_attention_gpu.py, for one and two row blocks per wave, every padded
 head size, and the qkv bias folded in.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import gptc
-from test_attention_gpu import compare_with_oracle
+from test_attention_gpu import check, compare_with_oracle, qkv_inputs
 from test_gpt2_gpu import self_attention_vs_oracle
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +54,48 @@ def test_slabs_are_deterministic(rt):
         rt.free(d)
         layer.free()
     assert all(np.array_equal(a, b) for a, b in zip(*seen))
+
+
+def shifted(rt, shape, shift):
+    """A tensor `shift` floats into a buffer (4-byte alignment only), and the buffer."""
+    n = int(np.prod(shape))
+    buf = rt.empty((n + shift,))
+    v = gptc.Tensor()
+    ctypes.memmove(ctypes.byref(v), buf, ctypes.sizeof(v))
+    v.t = ctypes.cast(ctypes.cast(buf.contents.t, ctypes.c_void_p).value + 4 * shift, ctypes.POINTER(ctypes.c_float))
+    v.ndims, v.length = len(shape), n
+    for i, d in enumerate(shape):
+        v.shape[i] = d
+    return ctypes.pointer(v), buf
+
+
+@pytest.mark.parametrize("B,T,C,H,shift", [
+    (4, 333, 768, 12, 0), (2, 1000, 768, 12, 0), (1, 650, 1600, 25, 0),   # heads of 64
+    (2, 1000, 960, 20, 0), (5, 200, 384, 24, 0),                          # of 48 and 16
+    (5, 208, 1536, 16, 0), (8, 200, 1280, 10, 0),                         # of 96 and 128
+    (2, 140, 128, 2, 1), (1, 333, 96, 2, 1), (1, 70, 256, 2, 1),          # gradients that are not 16-byte aligned
+])
+def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
+    """A backward that the slabs do not serve reads the forward's P' in halves of 32 queries, rows past T among them
+    (T ends in the first 16 rows of a half here).  The state is NaN before the forward: a row that it leaves out would
+    reach dK and dV as 0 * NaN."""
+    print(f"case halves B={B} T={T} C={C} H={H} shift={shift}", flush=True)
+    assert 0 < T % 32 <= 16
+    x, dy = qkv_inputs(rt, B, T, C)
+    lib = rt.lib
+    xt, dyt = rt.from_numpy(x), rt.from_numpy(dy)
+    mask = rt.from_numpy(np.tril(np.ones((T, T), np.float32)))
+    state = rt.empty((int(lib.gptc_attention_state_floats(B, T, C, H)),))
+    lib.fill_tensor_data_cuda(state, ctypes.c_float(np.nan))
+    yt = rt.empty((B, T, C))
+    caches = (gptc.TensorP * 4)(xt, yt, rt.empty((B, H, T)), state)
+    lib.attention_forward_cuda_kernel(xt, mask, H, caches, yt)
+    y = rt.to_numpy(yt)
+    dout, buf = shifted(rt, (B, T, 3 * C), shift)
+    lib.attention_backward_cuda_kernel(dyt, caches, H, dout)
+    d = rt.to_numpy(buf)[shift:].reshape(B, T, 3 * C)
+    for t in (xt, dyt, mask, yt, buf, caches[2], caches[3]):
+        rt.free(t)
+    y_ref, q, k, v, att = oracle.forward(x, H)
+    check("y", y, y_ref)
+    check("dqkv", d, oracle.backward(dy, H, q, k, v, att))
