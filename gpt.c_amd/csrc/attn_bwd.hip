@@ -1415,6 +1415,8 @@ void launch_attn_bwd(const BwdParams &p_in, hipStream_t stream, const hipEvent_t
         attn_bwd_dkdv_kernel<false, false, false, 2 * kDPad><<<grid_k, block, 0, stream>>>(p);
     else if (p.vec)
         attn_bwd_dkdv_kernel<true, false, false><<<grid_k, block, 0, stream>>>(p);
+    else if (p.D == kDPad && p.nqt <= kShortHeadTiles)  // an aligned forward of short heads stored no P'
+        attn_bwd_dkdv_kernel<false, false, true><<<grid_k, block, 0, stream>>>(p);
     else
         attn_bwd_dkdv_kernel<false, false, false><<<grid_k, block, 0, stream>>>(p);
     hipCheck(hipGetLastError());

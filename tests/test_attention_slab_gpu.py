@@ -69,18 +69,8 @@ def shifted(rt, shape, shift):
     return ctypes.pointer(v), buf
 
 
-@pytest.mark.parametrize("B,T,C,H,shift", [
-    (4, 333, 768, 12, 0), (2, 1000, 768, 12, 0), (1, 650, 1600, 25, 0),   # heads of 64
-    (2, 1000, 960, 20, 0), (5, 200, 384, 24, 0),                          # of 48 and 16
-    (5, 208, 1536, 16, 0), (8, 200, 1280, 10, 0),                         # of 96 and 128
-    (2, 140, 128, 2, 1), (1, 333, 96, 2, 1), (1, 70, 256, 2, 1),          # gradients that are not 16-byte aligned
-])
-def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
-    """A backward that the slabs do not serve reads the forward's P' in halves of 32 queries, rows past T among them
-    (T ends in the first 16 rows of a half here).  The state is NaN before the forward: a row that it leaves out would
-    reach dK and dV as 0 * NaN."""
-    print(f"case halves B={B} T={T} C={C} H={H} shift={shift}", flush=True)
-    assert 0 < T % 32 <= 16
+def prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift):
+    """Forward into a state that is NaN throughout, then backward into gradients `shift` floats into their buffer."""
     x, dy = qkv_inputs(rt, B, T, C)
     lib = rt.lib
     xt, dyt = rt.from_numpy(x), rt.from_numpy(dy)
@@ -99,3 +89,25 @@ def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
     y_ref, q, k, v, att = oracle.forward(x, H)
     check("y", y, y_ref)
     check("dqkv", d, oracle.backward(dy, H, q, k, v, att))
+
+
+@pytest.mark.parametrize("B,T,C,H,shift", [
+    (4, 333, 768, 12, 0), (2, 1000, 768, 12, 0), (1, 650, 1600, 25, 0),   # heads of 64
+    (2, 1000, 960, 20, 0), (5, 200, 384, 24, 0),                          # of 48 and 16
+    (5, 208, 1536, 16, 0), (8, 200, 1280, 10, 0),                         # of 96 and 128
+    (2, 140, 128, 2, 1), (1, 333, 96, 2, 1), (1, 70, 256, 2, 1),          # gradients that are not 16-byte aligned
+])
+def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
+    """A backward that the slabs do not serve reads the forward's P' in halves of 32 queries, rows past T among them
+    (T ends in the first 16 rows of a half here).  The state is NaN before the forward: a row that it leaves out would
+    reach dK and dV as 0 * NaN."""
+    print(f"case halves B={B} T={T} C={C} H={H} shift={shift}", flush=True)
+    assert 0 < T % 32 <= 16
+    prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift)
+
+
+@pytest.mark.parametrize("B,T,C,H", [(2, 17, 192, 3), (1, 64, 64, 1), (2, 100, 256, 4), (1, 128, 128, 2)])
+def test_unaligned_gradients_of_short_heads(rt, oracle, B, T, C, H):
+    """Heads of 64 up to 128 rows keep no P': the backward into gradients without 16-byte rows recomputes it too."""
+    print(f"case short unaligned B={B} T={T} C={C} H={H}", flush=True)
+    prefilled_state_vs_oracle(rt, oracle, B, T, C, H, 1)
