@@ -2,8 +2,8 @@
 // matrix cores.  No counterpart in gpt.c, whose GEMMs are cuBLAS calls
 // (kernels/src/cuda/Linear.cu:40-95).
 //
-// A float is the exact sum of three bf16 values (8 + 8 + 8 significant bits,
-// each part the rest rounded to nearest).  Of the nine products of two such
+// A float (from 2^-110 on) is the exact sum of three bf16 values (8 + 8 + 8
+// significant bits, each part the rest rounded to nearest).  Of the nine products of two such
 // sums, the six of relative order 2^0, 2^-8 and 2^-16 are formed; what is left
 // out is at most 3 x 2^-26 of a product, under half a rounding of the fp32
 // product.  A bf16 product is exact in the matrix core's fp32 sum, and
@@ -17,7 +17,15 @@
 // 32 terms sums its twelve products into a fresh accumulator, smallest first,
 // and the step's sum is added to the tile with a rounded fp32 add; every
 // second step forms -A B and is subtracted, which cancels what shift is
-// left.  Relative error against 64 bits (2-norm, normal inputs), this kernel
+// left.
+//
+// Range.  bf16 ends at 2^-133, so the parts of a float below 2^-110 would lose its
+// last bits.  Both operands are therefore split times 2^24 (exact: the last bit of
+// the smallest normal float is 2^-149), and a step's sum comes back times 2^-48 in
+// the add that takes it into the tile.  Floats of 2^104 and more, and sums of a step
+// past 2^80, overflow on the way: those blocks are formed again in fp32.
+//
+// Relative error against 64 bits (2-norm, normal inputs), this kernel
 // and rocBLAS's fp32 one: K = 768 1.0e-7 and 5.0e-7, 3072 1.9e-7 and 9.7e-7,
 // 8192 3e-7 and 1.6e-6; mean error under 2e-9 at K = 768 and 3072.
 //
@@ -57,6 +65,8 @@ constexpr int kBK = 32;      // reduction terms per step
 constexpr int kPlanes = 3;   // bf16 parts of a float
 constexpr int kPad = 2;      // 16-byte chunks of padding per row of chunks
 constexpr int kThreads = 256;
+constexpr float kScale = 0x1p24f;      // of either operand as it is split
+constexpr float kUnscale = 0x1p-48f;   // of a step's sum
 
 template <int N>
 using IntC = std::integral_constant<int, N>;
@@ -79,7 +89,7 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
 __device__ __forceinline__ float low_bf16(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float high_bf16(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
-// x, y = sum of their three bf16 parts, exactly.
+// x, y = sum of their three bf16 parts, exactly where their last bits are 2^-133 or more.
 __device__ __forceinline__ void split2(float x, float y, uint32_t (&p)[kPlanes]) {
     p[0] = pack_bf16(x, y);
     const float x1 = x - low_bf16(p[0]), y1 = y - high_bf16(p[0]);
@@ -191,7 +201,8 @@ struct Operand {
                     }
         }
     }
-    __device__ __forceinline__ void store(u32x4 *lds, int tid, float sign) const {
+    // scale: +-kScale, the step's sign in one operand
+    __device__ __forceinline__ void store(u32x4 *lds, int tid, float scale) const {
         if (KC) {
             const int kg = tid & 3;
 #pragma unroll
@@ -201,7 +212,7 @@ struct Operand {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     uint32_t p[kPlanes];
-                    split2(sign * v[8 * i + 2 * e], sign * v[8 * i + 2 * e + 1], p);
+                    split2(scale * v[8 * i + 2 * e], scale * v[8 * i + 2 * e + 1], p);
 #pragma unroll
                     for (int q = 0; q < kPlanes; ++q) c[q][e] = p[q];
                 }
@@ -218,8 +229,8 @@ struct Operand {
                     const int m = MV * ((lane >> 1) + 32 * i) + e;
                     const float *x = v + 4 * MV * i + e;
                     uint32_t a[kPlanes], b[kPlanes];
-                    split2(sign * x[0], sign * x[MV], a);
-                    split2(sign * x[2 * MV], sign * x[3 * MV], b);
+                    split2(scale * x[0], scale * x[MV], a);
+                    split2(scale * x[2 * MV], scale * x[3 * MV], b);
 #pragma unroll
                     for (int q = 0; q < kPlanes; ++q)
                         half[2 * ((4 * q + kg) * kRowChunks + row_slot(m)) + (lane & 1)] = u32x2{a[q], b[q]};
@@ -239,8 +250,9 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
                                                    0, 0);
 }
 
-// An infinity splits into inf - inf: a block that is not finite is formed again
-// from the floats themselves.  Ab, Bb: the operands from the tile's first row
+// An infinity (or a float or a step's sum that the scale takes past the largest)
+// splits into inf - inf: a block that is not finite is formed again from the
+// floats themselves.  Ab, Bb: the operands from the tile's first row
 // on; m, n: the block's first row and column in the tile.
 template <bool TA, bool TB>
 __device__ __forceinline__ void redo_if_not_finite(const Args &a, const float *Ab, const float *Bb, int m, int n,
@@ -353,8 +365,8 @@ split_gemm_kernel(const Args a) {
                 pb[d].mask(k_end - kd, tid);
             }
             __syncthreads();
-            pa[d].store(a_lds, tid, sign);
-            pb[d].store(b_lds, tid, 1.0f);
+            pa[d].store(a_lds, tid, sign * kScale);
+            pb[d].store(b_lds, tid, kScale);
             __syncthreads();
             // Past the end these read nothing (or terms that no step uses).
             pa[d].load(Ab, a.lda, rows_a, kd + DEPTH * kBK, k_end, tid);
@@ -387,7 +399,7 @@ split_gemm_kernel(const Args a) {
 #pragma unroll
                 for (int j = 0; j < NN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(sign, t[j][r], acc[i][j][r]);
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(sign * kUnscale, t[j][r], acc[i][j][r]);
             }
             sign = -sign;
         }
@@ -443,14 +455,14 @@ struct WaveOperand {
             for (int e = 0; e < 4; ++e)
                 if ((KC ? 4 * (lane & 3) + e : 8 * (lane >> 5) + 4 * (lane & 1) + i) >= left) v[4 * i + e] = 0.0f;
     }
-    __device__ __forceinline__ void store(u32x2 *lds, int lane, float sign) const {
+    __device__ __forceinline__ void store(u32x2 *lds, int lane, float scale) const {
         const int kg = KC ? (lane >> 1) & 1 : lane >> 5, half = lane & 1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int m = KC ? (lane >> 2) + 16 * i : 4 * ((lane >> 1) & 15) + i;
             uint32_t a[kPlanes], b[kPlanes];
-            split2(sign * (KC ? v[4 * i] : v[i]), sign * (KC ? v[4 * i + 1] : v[4 + i]), a);
-            split2(sign * (KC ? v[4 * i + 2] : v[8 + i]), sign * (KC ? v[4 * i + 3] : v[12 + i]), b);
+            split2(scale * (KC ? v[4 * i] : v[i]), scale * (KC ? v[4 * i + 1] : v[4 + i]), a);
+            split2(scale * (KC ? v[4 * i + 2] : v[8 + i]), scale * (KC ? v[4 * i + 3] : v[12 + i]), b);
 #pragma unroll
             for (int q = 0; q < kPlanes; ++q)
                 lds[2 * ((2 * q + kg) * kWRows + row_slot(m)) + half] = u32x2{a[q], b[q]};
@@ -501,8 +513,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 pa[d].mask(k_end - kd, lane);
                 pb[d].mask(k_end - kd, lane);
             }
-            pa[d].store(reinterpret_cast<u32x2 *>(a_lds), lane, sign);
-            pb[d].store(reinterpret_cast<u32x2 *>(b_lds), lane, 1.0f);
+            pa[d].store(reinterpret_cast<u32x2 *>(a_lds), lane, sign * kScale);
+            pb[d].store(reinterpret_cast<u32x2 *>(b_lds), lane, kScale);
             const int next = min(kd + kDepth * NW * kWK, k_end);
             pa[d].load(Ab, a.lda, rows_a, next, k_end, lane);
             pb[d].load(Bb, a.ldb, rows_b, next, k_end, lane);
@@ -531,7 +543,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(sign, t[j][r], acc[i][j][r]);
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(sign * kUnscale, t[j][r], acc[i][j][r]);
             }
             sign = -sign;
         }

@@ -144,3 +144,25 @@ def test_infinities_and_large_values(rt, case):
     cols = [c for c in range(fin) if c not in (7, 1, 819, 5)]
     check("dW, other columns", dW[:, cols], g.astype(np.float64).T, x[:, cols].astype(np.float64), 1.0)
     assert not np.isfinite(dW[:, [7, 1, 819]]).any()
+
+
+@pytest.mark.parametrize("ex,ew", [(-114, 60), (-118, 60), (-125, 90), (60, -114), (90, -125), (-60, -60)])
+def test_tiny_operands_keep_their_bits(rt, case, ex, ew):
+    """Normal floats down to the smallest keep all 24 bits (bf16 has nothing below 2^-133, so unscaled parts of floats
+    below 2^-110 would lose them); values of 2^ex times ordinary ones against 2^ew, the same bound as elsewhere."""
+    print(f"case tiny ex={ex} ew={ew}", flush=True)
+    rng = np.random.default_rng(7)
+    rows, fin, fout = 1000, 1201, 1100
+    scale = lambda a, e: np.ldexp(np.where(np.abs(a) < 1, np.copysign(np.float32(1), a), a), e).astype(np.float32)  # noqa: E731
+    x, W, g = scale(rnd(rng, rows, fin), ex), scale(rnd(rng, fout, fin), ew), scale(rnd(rng, rows, fout), ex)
+    y, dx, _, _ = linear(rt, case(), x, W, np.zeros(fout, np.float32), g)
+    X, W64, G = (np.ldexp(v.astype(np.float64), -e) for v, e in ((x, ex), (W, ew), (g, ex)))
+    check("y", np.ldexp(y, -ex - ew), X, W64.T)
+    check("dx", np.ldexp(dx, -ex - ew), G, W64)
+    # dW: g of 2^ex against x of 2^ew, onto zeros
+    x2 = scale(rnd(rng, rows, fin), ew)
+    c = case()
+    tg, tx, tW = c(g), c(x2), c(W)
+    dW, db, dx2 = c(np.zeros((fout, fin), np.float32)), c(np.zeros(fout, np.float32)), c(np.zeros((rows, fin), np.float32))
+    rt.lib.linear_backward_cuda_kernel(tg[0], tx[0], tW[0], dW[0], db[0], dx2[0])
+    check("dW", np.ldexp(c.get(dW, (fout, fin)), -ex - ew), G.T, np.ldexp(x2.astype(np.float64), -ew))
