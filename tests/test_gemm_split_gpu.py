@@ -121,6 +121,25 @@ def test_outputs_are_not_shifted(rt, case):
         assert abs(mean) < 1e-8, name
 
 
+@pytest.mark.parametrize("K", [7, 32, 96, 800])
+def test_sums_of_odd_step_counts_are_not_shifted(rt, case, K):
+    """One step, or an odd count of them, has no partner to cancel its truncation: the odd rows' and columns' signs
+    do, in sums over either.  Independent errors give sums of them the relative size that the outputs' own errors
+    have; twice that is asserted (a shift shows 8 to 17 times at K = 16 and 32, and 3 to 5 at 96)."""
+    print(f"case odd steps K={K}", flush=True)
+    rng = np.random.default_rng(K)
+    rows, fout = 4096, 1024
+    x, W, b, g = rnd(rng, rows, K), rnd(rng, fout, K), np.zeros(fout, np.float32), rnd(rng, rows, fout)
+    y, _, _, _ = linear(rt, case(), x, W, b, g)
+    ref = x.astype(np.float64) @ W.astype(np.float64).T
+    err = y - ref
+    own = np.linalg.norm(err) / np.linalg.norm(ref)
+    for axis in (0, 1):
+        share = np.linalg.norm(err.sum(axis)) / np.linalg.norm(ref.sum(axis)) / own
+        print(f"  sums over axis {axis}: {share:.2f} of the outputs' error {own:.2e}")
+        assert share < 2, axis
+
+
 def test_infinities_and_large_values(rt, case):
     """An infinity (or a float that rounds up to one in bf16) splits into inf - inf; such blocks are formed again in
     fp32, so products that involve one are what fp32 gives, and all others stay exact to the bound."""
