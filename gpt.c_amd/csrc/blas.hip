@@ -249,6 +249,17 @@ void launch_saxpy(int64_t n, float alpha, const float *x, int incx, float *y, in
     hipCheck(hipGetLastError());
 }
 
+// Equal slices of the reduction of C += A^T B that rocBLAS computes as one batch: its tiles of 128 x 128
+// outputs leave most CUs idle over a long reduction.  At least 1024 terms each, and no more
+// tiles than two a CU.  us, unsliced / sliced: 64 x 64 outputs over 2048 terms 11 / 9, over 8192 22 / 11;
+// 512 x 512 over 2048 27 / 15; 1024 x 24 over 4096 35 / 14; 384 x 384 over 3072 17 / 18.
+int library_slices(int M, int N, int K) {
+    const int64_t tiles = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+    int S = 1;
+    while (S < 8 && tiles * S < 512 && K % (2 * S) == 0 && K / (2 * S) >= 1024) S *= 2;
+    return S;
+}
+
 }  // namespace
 
 void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
@@ -258,8 +269,21 @@ void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const flo
         gptc::launch_split_gemm(g, gptc_stream_checked());
         return;
     }
-    gptc_sgemm(trans_a, trans_b, M, N, K, 1.0f, A, lda, B, ldb, add == C ? 1.0f : 0.0f, C, N);
     if (M <= 0 || N <= 0) return;
+    const int S = trans_a && !trans_b ? library_slices(M, N, K) : 1;
+    if (S > 1) {
+        hipStream_t s = gptc_stream_checked();
+        const long long n = static_cast<long long>(M) * N;
+        const int k = K / S;
+        float *part = static_cast<float *>(alloc_cuda(static_cast<size_t>(n) * S * sizeof(float)));
+        colmajor_gemm_batched(rocblas_operation_none, rocblas_operation_transpose, N, M, k, 1.0f, B, ldb,
+                              static_cast<long long>(k) * ldb, A, lda, static_cast<long long>(k) * lda, 0.0f, part, N, n, S,
+                              "sgemm_strided_batched (slices)");
+        gptc::launch_sum_slices(part, bias, add, C, M, N, N, S, s);
+        free_cuda(part);
+        return;
+    }
+    gptc_sgemm(trans_a, trans_b, M, N, K, 1.0f, A, lda, B, ldb, add == C ? 1.0f : 0.0f, C, N);
     if (bias != nullptr) gptc::launch_bias_add(C, bias, M, N, gptc_stream_checked());
     if (add != nullptr && add != C) launch_saxpy(static_cast<int64_t>(M) * N, 1.0f, add, 1, C, 1);
 }

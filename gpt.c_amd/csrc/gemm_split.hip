@@ -638,11 +638,18 @@ constexpr Tile kTiles[] = {
     {64, 64, 4, 0.80f, 0.45f, 0.42f, 1.35f},
 };
 // Products of fewer multiply-adds without a bias or residual stay with rocBLAS, whose small
-// fp32 tiles start up faster (1024 x 768 x 768: 13 us against 17; 300 x 512 x 512: 8
-// against 11; from 2048 x 768 x 768, 1.2e9, on the two are level); with a bias its
-// second launch costs what that gains (Linear forward and backward of 64 rows,
-// 768 to 2304: 54.5 us on rocBLAS alone, 48.0 here alone, 44.5 with this line).
+// fp32 tiles start up faster (us, here / rocBLAS: x W^T 300 x 512 x 512 11 / 8.5, 512 x 768 x 768
+// 14.6 / 8.8; both gradients of the latter 28 / 21).  From here on to about 2e9
+// rocBLAS is still up to 1.4 times as fast (1024 x 768 x 768 18 / 14, 2496 x 768 x 768 31 / 24; level at
+// 3328 x 768 x 768, 1.96e9), but its chained sums are five times as far off (5e-7 against
+// 1e-7, relative), so the line is not drawn there.  With a bias its second launch costs
+// about what the start gains (x W^T + b: 512 x 768 x 768 14.5 / 12.4, 64 x 768 x 2304 11.8 / 16.9,
+// 8192 x 64 x 64 5.9 / 8.8), so those run here at any size.
 constexpr double kLibraryMacs = 6e8;
+// rocBLAS does not split the reduction of an A without transposition: from 4096 terms on its
+// chain is the time, whatever the outputs (g W, 8 x 64 outputs, here / rocBLAS: 4096 terms 14 / 25,
+// 8192 17 / 451, 50257 33 / 2726; 128 x 256: 18 / 20, 21 / 444; at 2304 terms 8 x 768 12 / 12).
+constexpr int kLibraryTerms = 4096;
 constexpr int kSmallTile = 3;  // the 64 x 64 tile of eight independent waves
 
 struct Plan {
@@ -715,6 +722,23 @@ void run_small(const SplitGemm &g, Args a, int slices, hipStream_t stream) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+}  // namespace
+
+void launch_sum_slices(const float *part, const float *bias, const float *add, float *C, int M, int N, int ldc, int S,
+                       hipStream_t stream) {
+    const int64_t n = static_cast<int64_t>(M) * N;
+    const bool vec = N % 4 == 0 && ldc % 4 == 0 && aligned16(C) && aligned16(add) && aligned16(bias);
+    const int64_t items = vec ? n / 4 : n;
+    const int blocks = static_cast<int>(std::min<int64_t>((items + kThreads - 1) / kThreads, 256 * 8));
+    if (vec)
+        split_reduce_kernel<f32x4><<<dim3(blocks), dim3(kThreads), 0, stream>>>(part, bias, add, C, n, N, ldc, S);
+    else
+        split_reduce_kernel<float><<<dim3(blocks), dim3(kThreads), 0, stream>>>(part, bias, add, C, n, N, ldc, S);
+    hipCheck(hipGetLastError());
+}
+
+namespace {
+
 void run_plan(const SplitGemm &g, const Plan &p, hipStream_t s) {
     const int64_t n = static_cast<int64_t>(g.M) * g.N;
     float *part = nullptr;
@@ -733,26 +757,18 @@ void run_plan(const SplitGemm &g, const Plan &p, hipStream_t s) {
         default: run_small(g, a, p.slices, s); break;
     }
     if (p.slices == 1) return;
-    const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.C) && aligned16(g.add) && aligned16(g.bias);
-    const int64_t items = vec ? n / 4 : n;
-    const int blocks = static_cast<int>(std::min<int64_t>((items + kThreads - 1) / kThreads, 256 * 8));
-    if (vec)
-        split_reduce_kernel<f32x4><<<dim3(blocks), dim3(kThreads), 0, s>>>(part, g.bias, g.add, g.C, n, g.N, g.ldc,
-                                                                           p.slices);
-    else
-        split_reduce_kernel<float><<<dim3(blocks), dim3(kThreads), 0, s>>>(part, g.bias, g.add, g.C, n, g.N, g.ldc,
-                                                                           p.slices);
-    hipCheck(hipGetLastError());
+    launch_sum_slices(part, g.bias, g.add, g.C, g.M, g.N, g.ldc, p.slices, s);
     free_cuda(part);
 }
 
 }  // namespace
 
 bool split_gemm_serves(const SplitGemm &g) {
-    constexpr int kMaxLd = 1 << 22;  // a tile's offsets (256 rows) fit 32 bits
+    constexpr int kMaxLd = 1 << 22;  // a tile's offsets (128 rows) fit 32 bits
     if (g.M <= 0 || g.N <= 0 || g.K <= 0 || (g.trans_a && g.trans_b) || g.lda >= kMaxLd || g.ldb >= kMaxLd) return false;
     const double macs = static_cast<double>(g.M) * g.N * g.K;
-    return g.bias != nullptr || (g.add != nullptr && g.add != g.C) || macs >= kLibraryMacs;
+    return g.bias != nullptr || (g.add != nullptr && g.add != g.C) || macs >= kLibraryMacs ||
+           (!g.trans_a && g.K >= kLibraryTerms);
 }
 
 void launch_split_gemm(const SplitGemm &g, hipStream_t stream) { run_plan(g, choose(g), stream); }

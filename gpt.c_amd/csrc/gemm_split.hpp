@@ -24,4 +24,9 @@ bool split_gemm_serves(const SplitGemm &g);
 
 void launch_split_gemm(const SplitGemm &g, hipStream_t stream);
 
+// C (M x N, rows of ldc) = the sum of the S products in part (M x N each, without gaps, one
+// after the other; 16-byte aligned), in that order, (+ bias) (+ add, which may be C).
+void launch_sum_slices(const float *part, const float *bias, const float *add, float *C, int M, int N, int ldc, int S,
+                       hipStream_t stream);
+
 }  // namespace gptc

@@ -105,6 +105,29 @@ def test_linear_against_float64(rt, case, rows, fin, fout, shift):
         check("dW", dW, G.T, X, 1.0)
 
 
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 64, 4096), (8, 96, 50257), (33, 70, 8191), (130, 64, 16385),      # dx: long reductions
+    (2048, 64, 64), (4096, 77, 30), (8192, 128, 96), (3000, 200, 60), (2050, 64, 33),  # dW: sliced, and rows that are not
+    (2048, 512, 512),
+])
+def test_long_reductions_of_small_products(rt, case, rows, fin, fout):
+    """Below the size at which every product runs here: dx over 4096 features and more does as well, and a weight
+    gradient over 2048 rows and more is cut into slices of at least 1024 (2-norm error of a chain of K fp32 sums of
+    independent terms: about sqrt(K) 2^-25, 8e-7 at the 1024 - 2047 rows of a slice; 2e-6 is asserted)."""
+    print(f"case long rows={rows} in={fin} out={fout}", flush=True)
+    rng = np.random.default_rng(rows + fout)
+    x, W, b, g = rnd(rng, rows, fin), rnd(rng, fout, fin), rnd(rng, fout), rnd(rng, rows, fout)
+    assert rows * fin * fout < 6e8
+    _, dx, dW, _ = linear(rt, case(), x, W, b, g)
+    X, W64, G = (v.astype(np.float64) for v in (x, W, g))
+    if fout >= 4096:
+        check("dx", dx, G, W64)
+    ref = G.T @ X + 1.0
+    rel = np.linalg.norm(dW - ref) / np.linalg.norm(ref)
+    print(f"  dW: 2-norm {rel:.2e}")
+    assert rel <= 2e-6
+
+
 def test_outputs_are_not_shifted(rt, case):
     """The matrix core truncates towards minus infinity; the alternating signs of the steps cancel it.  The mean
     error over 8192 x 768 outputs is then a sample mean of errors of 2e-7 x the outputs' size: 1e-8 is 100 of its
