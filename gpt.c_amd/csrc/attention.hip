@@ -483,10 +483,14 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
             p.dbq_part = cache[3]->t + st.dbq;
             p.dbkv_part = cache[3]->t + st.dbkv;
             p.C = d.C;
-            if (p.slab) {
+            if (p.slab && lse_only) {
                 db_part = static_cast<float *>(
                     alloc_cuda(static_cast<size_t>(d.B) * gptc::slab_count(p) * 3 * d.C * sizeof(float)));
                 p.dbq_part = db_part;
+            } else if (p.slab) {
+                // In the P' blocks, which the slabs do not read: 2048 nqt (nqt + 1) floats a head for at
+                // most 4 nqt rows of 192.
+                p.dbq_part = cache[3]->t + st.p;
             }
         }
     }
@@ -497,8 +501,8 @@ void backward_impl(const tensor_t *global_grad, tensor_t **cache, const tensor_t
     if (bias != nullptr) {
         const int nqt = (d.T + 63) / 64, nkb = (d.T + 127) / 128;
         if (folded && p.slab) {
-            gptc::launch_add_column_partials(db_part, db->t, d.B * gptc::slab_count(p), 3 * d.C, s);
-            free_cuda(db_part);
+            gptc::launch_add_column_partials(p.dbq_part, db->t, d.B * gptc::slab_count(p), 3 * d.C, s);
+            if (db_part != nullptr) free_cuda(db_part);
         } else if (folded) {
             // db += the per-block column sums, in a fixed order.
             gptc::launch_add_column_partials(p.dbq_part, db->t, d.B * nqt, d.C, s);

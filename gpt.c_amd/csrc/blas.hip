@@ -271,7 +271,7 @@ void gptc_linear_gemm(bool trans_a, bool trans_b, int M, int N, int K, const flo
     }
     if (M <= 0 || N <= 0) return;
     const int S = trans_a && !trans_b ? library_slices(M, N, K) : 1;
-    if (S > 1) {
+    if (S > 1 && !gptc_stream_capturing()) {
         hipStream_t s = gptc_stream_checked();
         const long long n = static_cast<long long>(M) * N;
         const int k = K / S;

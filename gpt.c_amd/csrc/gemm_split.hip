@@ -652,6 +652,8 @@ constexpr double kLibraryMacs = 6e8;
 constexpr int kLibraryTerms = 4096;
 constexpr int kSmallTile = 3;  // the 64 x 64 tile of eight independent waves
 
+constexpr int kMaxSlices = 32;
+
 struct Plan {
     int tile, slices, slice_k;
 };
@@ -675,12 +677,12 @@ float plan_us(int tile, const SplitGemm &g, int S) {
     return S == 1 ? us : us + 4.0f + 0.1f * S + (S + 2) * (static_cast<float>(g.M) * g.N * 4e-6f / 4.5f);
 }
 
-Plan choose(const SplitGemm &g) {
+Plan choose(const SplitGemm &g, int max_slices) {
     const int steps = (g.K + kBK - 1) / kBK;
     Plan best{0, 1, 0};
     float best_us = INFINITY;
     for (int t = 0; t <= kSmallTile; ++t)
-        for (int S = 1; S <= 32 && S <= steps; ++S) {
+        for (int S = 1; S <= max_slices && S <= steps; ++S) {
             const float us = plan_us(t, g, S);
             if (us < best_us) {
                 best_us = us;
@@ -771,6 +773,10 @@ bool split_gemm_serves(const SplitGemm &g) {
            (!g.trans_a && g.K >= kLibraryTerms);
 }
 
-void launch_split_gemm(const SplitGemm &g, hipStream_t stream) { run_plan(g, choose(g), stream); }
+void launch_split_gemm(const SplitGemm &g, hipStream_t stream) {
+    Plan p = choose(g, kMaxSlices);
+    if (p.slices > 1 && gptc_stream_capturing()) p = choose(g, 1);
+    run_plan(g, p, stream);
+}
 
 }  // namespace gptc

@@ -22,6 +22,7 @@ struct SplitGemm {
 // within their 32-bit tile offsets, a layout they are built for).
 bool split_gemm_serves(const SplitGemm &g);
 
+// Under graph capture the reduction stays whole: slices would take a block of the pool.
 void launch_split_gemm(const SplitGemm &g, hipStream_t stream);
 
 // C (M x N, rows of ldc) = the sum of the S products in part (M x N each, without gaps, one

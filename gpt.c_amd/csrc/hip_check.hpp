@@ -20,6 +20,11 @@ inline void hip_check(hipError_t err, const char *file, int line) {
 // (fatal if runtime_init_cuda() has not run).
 hipStream_t gptc_stream_checked();
 
+// Whether that stream is being captured into a graph.  A graph's replays use the pool's blocks
+// that its launches took for scratch after those have gone to someone else: entry points that
+// can do without scratch do so under capture.
+bool gptc_stream_capturing();
+
 // The serial of the live alloc_cuda block starting at ptr (0 if it is none):
 // new at each allocation of the block and at each write of the library's
 // tensor data ops into it (gptc_block_written).

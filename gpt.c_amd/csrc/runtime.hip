@@ -78,6 +78,12 @@ hipStream_t gptc_stream_checked() {
     return g_stream;
 }
 
+bool gptc_stream_capturing() {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    hipCheck(hipStreamIsCapturing(gptc_stream_checked(), &st));
+    return st != hipStreamCaptureStatusNone;
+}
+
 extern "C" void runtime_init_cuda(void) {
     if (g_ready) return;
     int count = 0;
