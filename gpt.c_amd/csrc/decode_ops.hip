@@ -380,20 +380,29 @@ void run_ln_held(const RowsArgs &a, hipStream_t s) {
     }
 }
 
+// The compile-time row counts, for rows that are no whole vectors too (a token of 4 layers,
+// C = 771, with a run-time count, with 8 rows always, now: 1 row 265 / 271 / 227 us, 3 rows 322 / 269 / 241;
+// C = 342, 1 row 144 / 142 / 122).
+template <bool kVec, bool kLN, int kOuts, int kPer>
+void launch_rows_of(const RowsArgs &a, hipStream_t s) {
+    const dim3 grid((a.out_f + kOuts * kPer - 1) / (kOuts * kPer));
+    if (a.rows == 1)
+        linear_rows_kernel<kVec, kLN, kOuts, kPer, 1><<<grid, dim3(kThreads), 0, s>>>(a);
+    else if (a.rows == 2)
+        linear_rows_kernel<kVec, kLN, kOuts, kPer, 2><<<grid, dim3(kThreads), 0, s>>>(a);
+    else if (a.rows <= 4)
+        linear_rows_kernel<kVec, kLN, kOuts, kPer, 4><<<grid, dim3(kThreads), 0, s>>>(a);
+    else
+        linear_rows_kernel<kVec, kLN, kOuts, kPer, kMaxRows><<<grid, dim3(kThreads), 0, s>>>(a);
+    hipCheck(hipGetLastError());
+}
+
 template <bool kLN, int kOuts, int kPer>
 void launch_rows(const RowsArgs &a, bool vec, hipStream_t s) {
-    const dim3 grid((a.out_f + kOuts * kPer - 1) / (kOuts * kPer));
-    if (!vec)
-        linear_rows_kernel<false, kLN, kOuts, kPer, kMaxRows><<<grid, dim3(kThreads), 0, s>>>(a);
-    else if (a.rows == 1)
-        linear_rows_kernel<true, kLN, kOuts, kPer, 1><<<grid, dim3(kThreads), 0, s>>>(a);
-    else if (a.rows == 2)
-        linear_rows_kernel<true, kLN, kOuts, kPer, 2><<<grid, dim3(kThreads), 0, s>>>(a);
-    else if (a.rows <= 4)
-        linear_rows_kernel<true, kLN, kOuts, kPer, 4><<<grid, dim3(kThreads), 0, s>>>(a);
+    if (vec)
+        launch_rows_of<true, kLN, kOuts, kPer>(a, s);
     else
-        linear_rows_kernel<true, kLN, kOuts, kPer, kMaxRows><<<grid, dim3(kThreads), 0, s>>>(a);
-    hipCheck(hipGetLastError());
+        launch_rows_of<false, kLN, kOuts, kPer>(a, s);
 }
 
 // Narrow outputs (under 1024 features) split each dot product over the 4

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     (1, 4, 260), (7, 4, 260),    # 65 vectors a row
     (1, 16, 1024), (6, 16, 1024), (2, 16, 1024),
     (1, 13, 1040), (8, 13, 1040),
-    (4, 3, 342),                 # rows that are no whole vectors
+    (4, 3, 342), (1, 3, 342), (2, 3, 342), (7, 3, 342), (1, 3, 771), (3, 3, 771),  # rows that are no whole vectors
 ])
 def test_decode_rows(rt, B, H, C):
     print(f"case decode rows B={B} H={H} C={C}", flush=True)
