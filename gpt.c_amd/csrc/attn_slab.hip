@@ -97,8 +97,24 @@ __device__ __forceinline__ f32x4 take_sums(const f32x4 (*lds)[R][NB][64], int i,
     return v;
 }
 
+// x . b of row i16 of a block (b: the head's values of one bias), on every lane of the row's
+// column; D = 64 NC / 4 only.
+template <int NC>
+__device__ __forceinline__ float dot_bias(const f32x4 (&x)[NC], const float *b, int g) {
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const f32x4 v = at4(b + 16 * c + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = fmaf(x[c][e], v[e], s);
+    }
+    return sum4_rows(s);
+}
+
 // y, the log-sum-exp, P' and m of R blocks of queries; wave w takes the 64-key tiles
-// w, w + 4, ...  DP: the padded head size; BIAS: the qkv bias joins the rows.
+// w, w + 4, ...  DP: the padded head size; BIAS: the qkv bias is added here.  It joins the
+// slab's own rows only: (q + qb) . (k + kb) starts from the row's (q + qb) . kb, and the
+// probabilities' sum of v + vb is that of v, and vb.
 template <int DP, int R, bool BIAS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 64 ? 2 : 1, DP == 64 ? 2 : 1))) void
 attn_fwd_slab_kernel(const FwdParams a) {
@@ -120,7 +136,7 @@ attn_fwd_slab_kernel(const FwdParams a) {
     const HeadRows<DP> k_rows(a.k.p + b * a.k.sb + h * a.k.sh, T, a.k.st, D);
     const HeadRows<DP> v_rows(a.v.p + b * a.v.sb + h * a.v.sh, T, a.v.st, D);
     f32x4 qr[R][NC], acc[R][NB];
-    float m_run[R], l_run[R];
+    float m_run[R], l_run[R], s0[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         q_rows.by_row(q0 + kBlock * i, g, i16, qr[i]);
@@ -128,6 +144,7 @@ attn_fwd_slab_kernel(const FwdParams a) {
 #pragma unroll
             for (int c = 0; c < NC; ++c) qr[i][c] += at4(a.qb + h * D + 16 * c + 4 * g);
         }
+        s0[i] = BIAS ? dot_bias(qr[i], a.kb + h * D, g) : 0.0f;
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[i][n] = zero4();
         m_run[i] = -INFINITY;
@@ -141,19 +158,11 @@ attn_fwd_slab_kernel(const FwdParams a) {
         for (int kb = 0; kb < 4; ++kb) k_rows.by_row(64 * kt + kBlock * kb, g, i16, kr[kb]);
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) v_rows.by_dim(64 * kt + kBlock * kb, g, i16, vr[kb]);
-        if (BIAS) {
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const f32x4 kb4 = at4(a.kb + h * D + 16 * c + 4 * g);
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) kr[kb][c] += kb4;
-            }
-        }
         f32x4 sc[R][4];
 #pragma unroll
         for (int i = 0; i < R; ++i)
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb) sc[i][kb] = zero4();
+            for (int kb = 0; kb < 4; ++kb) sc[i][kb] = f32x4{s0[i], s0[i], s0[i], s0[i]};
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -210,23 +219,17 @@ attn_fwd_slab_kernel(const FwdParams a) {
                 if (g == 0 && my_q < T) a.pm[(static_cast<uint32_t>(bh) * a.nqt + kt) * T + my_q] = m_use;
             }
         }
-        f32x4 vb4[NE];
-        if (BIAS) {
-#pragma unroll
-            for (int e = 0; e < NE; ++e) vb4[e] = at4(a.vb + h * D + 64 * e + 4 * i16);
-        }
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int e = 0; e < NE; ++e) {
-                    const f32x4 v = BIAS ? vr[kb][r][e] + vb4[e] : vr[kb][r][e];
+                for (int e = 0; e < NE; ++e)
 #pragma unroll
                     for (int i = 0; i < R; ++i)
 #pragma unroll
-                        for (int n = 0; n < 4; ++n) acc[i][4 * e + n] = mfma16(v[n], sc[i][kb][r], acc[i][4 * e + n]);
-                }
+                        for (int n = 0; n < 4; ++n)
+                            acc[i][4 * e + n] = mfma16(vr[kb][r][e][n], sc[i][kb][r], acc[i][4 * e + n]);
     }
 
     put_sums<R, NB>(sums, w, lane, acc);
@@ -258,7 +261,8 @@ attn_fwd_slab_kernel(const FwdParams a) {
         for (int e = 0; e < NE; ++e) {
             const int dim = 64 * e + 16 * g + 4 * w;
             if (dim >= D) continue;
-            const f32x4 v = take_sums<R, NB>(sums, i, e, w, lane, f) * inv;
+            f32x4 v = take_sums<R, NB>(sums, i, e, w, lane, f) * inv;
+            if (BIAS) v += at4(a.vb + h * D + dim);
             const size_t at = b * a.o.sb + static_cast<size_t>(my_q) * a.o.st + h * a.o.sh + dim;
             *reinterpret_cast<f32x4 *>(a.o.p + at) = v;
             if (a.o2 != nullptr) *reinterpret_cast<f32x4 *>(a.o2 + at) = v;
@@ -298,6 +302,12 @@ __device__ __forceinline__ void store_slab(const f32x4 (*sums)[R][DP / 16][64], 
     }
 }
 
+// BIAS: the qkv bias joins the slab's own rows only.  The products with the rows that stream by
+// start from the slab rows' products with their bias; dQ needs no k bias (a row of dS sums to
+// zero), and dK takes the q bias times the key's sum of dS at the end.  So the form with
+// the bias keeps the other's registers (adding the bias to the rows as they came spilled 14 of
+// them; us with its column sums' launch, then / now / without bias: 12 heads T = 1024 89 / 78 / 72, 3 heads
+// T = 2048 147 / 118 / 111; forward of the same 36.6 / 32.7 / 32.5, 42 / 36 / 36).
 template <int DP, int R, bool BIAS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 64 ? 2 : 1, DP == 64 ? 2 : 1))) void
 attn_bwd_slab_kernel(const BwdParams a) {
@@ -322,16 +332,6 @@ attn_bwd_slab_kernel(const BwdParams a) {
             for (int c = 0; c < NC; ++c) x[c] += at4(p + h * D + 16 * c + 4 * g);
         }
     };
-    auto bias2 = [&](const float *p, f32x4 (&x)[4][NE]) {
-        if (BIAS) {
-#pragma unroll
-            for (int e = 0; e < NE; ++e) {
-                const f32x4 v = at4(p + h * D + 64 * e + 4 * i16);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) x[r][e] += v;
-            }
-        }
-    };
     // rowsum(dO o O) of row i16 of a block, on every lane of the row's column.
     auto delta_of = [&](const f32x4 (&x)[NC], const f32x4 (&y)[NC]) {
         float s = 0.0f;
@@ -349,7 +349,7 @@ attn_bwd_slab_kernel(const BwdParams a) {
         const int slab = n_slabs - 1 - (rank >> 1), q0 = R * kBlock * slab;
         const int last = min(R * slab + R, n_blocks) - 1;
         f32x4 qr[R][NC], dor[R][NC], acc[R][NB];
-        float dl[R], lse2[R];
+        float dl[R], lse2[R], s0[R];
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const int row = q0 + kBlock * i;
@@ -359,6 +359,11 @@ attn_bwd_slab_kernel(const BwdParams a) {
             o_rows.by_row(row, g, i16, orow);
             dl[i] = delta_of(orow, dor[i]);
             bias1(a.qb, qr[i]);
+            s0[i] = 0.0f;
+            if (BIAS) {
+                s0[i] = dot_bias(qr[i], a.kb + h * D, g);
+                dl[i] -= dot_bias(dor[i], a.vb + h * D, g);
+            }
             // Rows past T: P = 0 (their dO rows are zero too).
             lse2[i] = row + i16 < T ? lse_h[min(row + i16, T - 1)] * kLog2e : INFINITY;
 #pragma unroll
@@ -372,11 +377,12 @@ attn_bwd_slab_kernel(const BwdParams a) {
         for (int kb = w; kb <= last; kb += kSlabWaves) {
             f32x4 k2[4][NE];
             k_rows.by_dim(kBlock * kb, g, i16, k2);
-            bias1(a.kb, k1);
-            bias1(a.vb, v1);
             f32x4 sc[R], dp[R];
 #pragma unroll
-            for (int i = 0; i < R; ++i) sc[i] = dp[i] = zero4();
+            for (int i = 0; i < R; ++i) {
+                sc[i] = f32x4{s0[i], s0[i], s0[i], s0[i]};
+                dp[i] = zero4();
+            }
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -389,7 +395,6 @@ attn_bwd_slab_kernel(const BwdParams a) {
             // The next block's rows (past the slab: rows that no step uses).
             k_rows.by_row(kBlock * (kb + kSlabWaves), g, i16, k1);
             v_rows.by_row(kBlock * (kb + kSlabWaves), g, i16, v1);
-            bias2(a.kb, k2);
 #pragma unroll
             for (int i = 0; i < R; ++i)
 #pragma unroll
@@ -415,12 +420,15 @@ attn_bwd_slab_kernel(const BwdParams a) {
     // blocks from the slab's first on.
     const int slab = rank >> 1, k0 = R * kBlock * slab;
     f32x4 kr[R][NC], vr[R][NC], acc_k[R][NB], acc_v[R][NB];
+    float s0[R], ds_sum[R];  // BIAS: the keys' (k + kb) . qb, and this lane's part of their sums of dS
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         k_rows.by_row(k0 + kBlock * i, g, i16, kr[i]);
         v_rows.by_row(k0 + kBlock * i, g, i16, vr[i]);
         bias1(a.kb, kr[i]);
         bias1(a.vb, vr[i]);
+        s0[i] = BIAS ? dot_bias(kr[i], a.qb + h * D, g) : 0.0f;
+        ds_sum[i] = 0.0f;
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc_k[i][n] = acc_v[i][n] = zero4();
     }
@@ -439,10 +447,12 @@ attn_bwd_slab_kernel(const BwdParams a) {
         for (int r = 0; r < 4; ++r) lse2[r] = lse_h[min(q0 + 4 * g + r, T - 1)];
         do_rows.by_dim(q0, g, i16, do2);
         q_rows.by_dim(q0, g, i16, q2);
-        bias1(a.qb, q1);
         f32x4 sc[R], dp[R];
 #pragma unroll
-        for (int i = 0; i < R; ++i) sc[i] = dp[i] = zero4();
+        for (int i = 0; i < R; ++i) {
+            sc[i] = f32x4{s0[i], s0[i], s0[i], s0[i]};
+            dp[i] = zero4();
+        }
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -455,7 +465,6 @@ attn_bwd_slab_kernel(const BwdParams a) {
         const float d1 = delta_of(o1, do1);
         q_rows.by_row(kBlock * (qb + kSlabWaves), g, i16, q1);
         do_rows.by_row(kBlock * (qb + kSlabWaves), g, i16, do1);
-        bias2(a.qb, q2);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             dl[r] = __shfl(d1, 4 * g + r, 64);
@@ -469,6 +478,7 @@ attn_bwd_slab_kernel(const BwdParams a) {
                 if (k0 + kBlock * i + i16 > q0 + 4 * g + r) p = 0.0f;
                 sc[i][r] = p;
                 dp[i][r] = p * (dp[i][r] - dl[r]);
+                if (BIAS) ds_sum[i] += dp[i][r];
             }
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -481,6 +491,20 @@ attn_bwd_slab_kernel(const BwdParams a) {
                 }
     }
     if (a.db != nullptr) part = a.dbq_part + (static_cast<size_t>(b) * n_slabs + slab) * 3 * a.C + a.C + h * D;
+    if (BIAS) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const float s = sum4_rows(ds_sum[i]);
+#pragma unroll
+            for (int e = 0; e < NE; ++e)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const f32x4 qb4 = at4(a.qb + h * D + 64 * e + 16 * g + 4 * r);
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) acc_k[i][4 * e + n][r] = fmaf(s, qb4[n], acc_k[i][4 * e + n][r]);
+                }
+        }
+    }
     put_sums<R, NB>(sums, w, lane, acc_k);
     __syncthreads();
     store_slab<DP, R>(sums, w, lane, a.scale, a.dk, b, h, k0, T, D, part);

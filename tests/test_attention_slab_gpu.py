@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import gptc
-from test_attention_gpu import check, compare_with_oracle, qkv_inputs
+from test_attention_gpu import check, compare_with_oracle, lse_fp64, qkv_inputs
 from test_gpt2_gpu import self_attention_vs_oracle
 
 pytestmark = pytest.mark.gpu
@@ -36,6 +36,35 @@ def test_slabs_with_qkv_bias(rt, oracle, B, T, C, H):
     """The bias added to the rows and its gradient from the slabs' column sums (one and two blocks per slab)."""
     print(f"case slab bias B={B} T={T} C={C} H={H}", flush=True)
     self_attention_vs_oracle(rt, oracle, B, T, C, H)
+
+
+@pytest.mark.parametrize("B,T,C,H", [
+    (1, 15, 64, 1), (1, 40, 128, 2), (2, 129, 128, 2), (3, 333, 192, 3),          # one block per slab
+    (1, 1009, 192, 3), (4, 200, 512, 8), (1, 640, 448, 7), (3, 321, 448, 7),      # two (350 tiles or more)
+])
+def test_slabs_with_a_large_qkv_bias(rt, oracle, B, T, C, H):
+    """Biases of the rows' own size through the entry points: y, the log-sum-exp, dqkv and db against the oracle on
+    the rows with the bias added, one backward of a head's q, k and v parts each."""
+    print(f"case slab large bias B={B} T={T} C={C} H={H}", flush=True)
+    x, dy = qkv_inputs(rt, B, T, C)
+    bias = rt.normal((3 * C,), 5)
+    lib = rt.lib
+    xt, dyt, bt = rt.from_numpy(x), rt.from_numpy(dy), rt.from_numpy(bias)
+    mask = rt.from_numpy(np.tril(np.ones((T, T), np.float32)))
+    yt, dout, db = rt.empty((B, T, C)), rt.empty((B, T, 3 * C)), rt.from_numpy(np.zeros(3 * C, np.float32))
+    caches = (gptc.TensorP * 4)(xt, yt, rt.empty((B, H, T)), rt.empty((int(lib.gptc_attention_state_floats(B, T, C, H)),)))
+    lib.gptc_attention_forward_qkv_bias(xt, bt, mask, H, caches, yt)
+    lib.gptc_attention_backward_qkv_bias(dyt, caches, bt, H, dout, db)
+    y, lse, d, dbias = rt.to_numpy(yt), rt.to_numpy(caches[2]), rt.to_numpy(dout), rt.to_numpy(db)
+    for t in (xt, dyt, bt, mask, yt, dout, db, caches[2], caches[3]):
+        rt.free(t)
+    y_ref, q, k, v, att = oracle.forward(x + bias, H)
+    d_ref = oracle.backward(dy, H, q, k, v, att)
+    check("y", y, y_ref)
+    check("lse", lse.reshape(B, H, T), lse_fp64(q, k))
+    check("dqkv", d, d_ref)
+    # Column sums of B T rows, each within the rows' own tolerance of independent sign.
+    check("db", dbias, d_ref.astype(np.float64).sum((0, 1)), 1e-4 * np.sqrt(B * T))
 
 
 def test_slabs_are_deterministic(rt):
