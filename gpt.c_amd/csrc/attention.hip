@@ -539,6 +539,26 @@ extern "C" long long gptc_attention_state_floats(int B, int T, int C, int n_head
     return forward_state(d, false, d.D == gptc::kDPad, &lse_only).total;
 }
 
+extern "C" int gptc_attention_slabs(int B, int T, int C, int n_heads) {
+    CHECK_ERROR(B < 0 || T < 0 || C < 0 || n_heads <= 0 || C % n_heads != 0,
+                "Expected B, T, C >= 0 and C divisible by n_heads > 0, but got B=%d, T=%d, C=%d, n_heads=%d.", B, T,
+                C, n_heads);
+    const Dims d{B, T, C, n_heads, C / n_heads};
+    if (B == 0 || T == 0 || C == 0) return 0;
+    FwdParams f{};
+    qkv_views(nullptr, d, f.q, f.k, f.v);
+    BwdParams b{};
+    qkv_views(nullptr, d, b.q, b.k, b.v);
+    b.o = b.dout = btc_view<HeadView>(static_cast<const float *>(nullptr), d);
+    f.B = b.B = d.B;
+    f.H = b.H = d.H;
+    f.T = b.T = d.T;
+    f.D = b.D = d.D;
+    f.nqt = b.nqt = (d.T + 63) / 64;
+    f.vec = b.vec = d.D % 4 == 0;
+    return (gptc::fwd_slab(f) ? 1 : 0) | (gptc::bwd_slab(b) ? 2 : 0);
+}
+
 extern "C" long long gptc_attention_set_state_limit(long long floats) {
     return g_state_limit.exchange(floats < 0 ? static_cast<long long>(INT32_MAX) : floats);
 }

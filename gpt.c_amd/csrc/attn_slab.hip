@@ -27,6 +27,7 @@
 // T = 333 64.7 / 32.6, B = 2 H = 8 T = 1024 D = 128 486 / 290, B = 1 H = 12 T = 1024
 // forward 56.1 / 31.2.
 #include <algorithm>
+#include <cmath>
 
 #include "attn_common.hpp"
 #include "attn_kernels.hpp"
@@ -525,42 +526,73 @@ bool rows_fit(int T, int D, std::initializer_list<uint32_t> strides) {
 
 namespace {
 
-// The rule that picks the slab kernels, from times measured on the MI355X (us).
-// tiles = B H nqt (nqt + 1) / 2, the 64 x 64 tiles below the diagonals.  The
-// slabs' time is fixed + per tile (their waves are many and short, so the sum of the
-// work sets it), with one or two blocks of rows per wave: two load half as much
-// per product, one makes twice the workgroups (r2_from: the tiles from which
-// two are faster).  The kernels on work lists and 128-row blocks take their
-// longest chain, chain0 + chain nqt, or the sum of the work, sum0 + sum tiles.
+// The rule that picks the slab kernels, from times measured on the MI355X (us; 1128 cases
+// of each direction, up to 22000 tiles, head sizes 32, 48, 64, 96 and 128, T = 16 to 2048, both sides
+// forced, heads of 64 with and without the bias).
+// tiles = B H nqt (nqt + 1) / 2, the 64 x 64 tiles below the diagonals.
+//
+// The slabs' workgroups come in rounds of 256 times the resident ones; a last round that
+// is partly empty costs `tail` of what is missing in it.  A workgroup takes as many steps of its four
+// waves as it has blocks on the other side, on average (blocks + 4) / 8: `one` us a step with
+// one block of rows per wave, start2 + `two` with two, which load half as much per product where
+// one makes twice the workgroups (r2_from: the tiles from which two are faster).  The
+// kernels on work lists and 128-row blocks take their longest chain, chain0 + chain nqt, or the
+// sum of the work, sum0 + sum tiles.
+//
+// Against the faster of the two at each shape the rule loses 0.4 % on average in the forward and 0.1 % in
+// the backward; a rule on tiles alone lost 1.3 and 0.8 %, and up to 55 % where the last round of
+// workgroups is nearly empty (130 heads of 128 T = 256 78 / 51).  Where it picks the slabs they are at most
+// 3 % slower but for 48 dims: forward 95 to 114 heads T = 333 to 384 5 and 6 %, backward 256 heads T = 64 24.9 / 22.6; and
+// 128 dims, backward 57 heads T = 333 134 / 128 us.
 struct SlabTimes {
-    float fixed, one, two, r2_from;
+    float fixed, one, start2, two, tail;
+    int resident;
+    float r2_from;
+    float per_tile;  // with every CU busy to the end: no less than fixed + this a tile
     float chain0, chain, sum0, sum;
 };
-// Forward, head sizes up to 64: 64 itself, and the others against the 32-row kernel.
-// Slab / other at 12 heads of 64: B = 1 T = 1024 31.2 / 56.1, B = 2 50 / 56, B = 8
-// T = 256 24 / 17; 48 dims B = 2 T = 1024 47.6 / 95.6, 32 dims 64 heads T = 1024 110 / 107.
-constexpr SlabTimes kFwd64{9, 12.5e-3f, 12.5e-3f, 1e9f, 2, 3.4f, 4, 9.4e-3f};
-constexpr SlabTimes kFwd32{9, 12.0e-3f, 12.0e-3f, 1e9f, 4, 5.8f, 4, 12.0e-3f};
-// Up to 128 dims: 16 heads of 128, T = 1024 62 / 155, 32 heads 124 / 156, 64 heads 245 / 183.
-constexpr SlabTimes kFwd128{6, 33e-3f, 26.5e-3f, 1000, 3, 9.6f, 4, 20.6e-3f};
-// Backward: 12 heads of 64, T = 1024 72 / 98, 24 heads 130 / 100; T = 600, 24 heads 58 / 66;
-// T = 200, 48 heads 28 / 33; 15 heads T = 333 20 / 41; T = 256, 96 heads 54 / 49.
-constexpr SlabTimes kBwd64{8, 52e-3f, 41e-3f, 350, 18, 5.0f, 10, 19.5e-3f};
-// 48 dims, 24 heads T = 1024 125 / 184; 32 dims, 96 heads T = 200 39 / 49, 64 heads T = 1024 290 / 235.
-constexpr SlabTimes kBwd32{8, 42e-3f, 38e-3f, 350, 8, 10.5f, 10, 26e-3f};
-// 16 heads of 128, T = 1024 230 / 330, 32 heads 409 / 339; 80 dims, 32 heads T = 300 59 / 107.
-constexpr SlabTimes kBwd128{12, 110e-3f, 96e-3f, 250, 8, 20.0f, 10, 46e-3f};
+// Slab / other: 12 heads of 64 B = 1 T = 1024 32 / 56, 24 heads 52 / 57, 33 heads 84 / 62, 20 heads T = 640 24 / 36,
+// 48 heads T = 256 17 / 17.
+constexpr SlabTimes kFwd64{4.4f, 6.8f, 0, 0, 0.45f, 2, 1e9f, 15.0e-3f, 1.55f, 3.71f, 6.2f, 10.8e-3f};
+// 48 dims 24 heads T = 1024 51 / 96, 66 heads 166 / 127; 120 heads T = 200 24 / 26, 220 heads 39 / 35.
+constexpr SlabTimes kFwd32{2.07f, 6.0f, 0, 0, 0.634f, 2, 1e9f, 14.0e-3f, 3.0f, 5.85f, 8.18f, 12.8e-3f};
+// 16 heads of 128, T = 1024 65 / 155, 33 heads 156 / 158, 48 heads 191 / 166; 120 heads T = 200 55 / 44.
+constexpr SlabTimes kFwd128{3.23f, 8.29f, 0.545f, 13.0f, 0.729f, 1, 1000, 28.5e-3f, 4.61f, 9.49f, 13.8f, 27.0e-3f};
+// 9 heads of 64 T = 1024 70 / 97, 16 heads 104 / 98; 22 heads T = 640 60 / 66; 57 heads T = 333 56 / 48; with the bias
+// 16 heads T = 1024 109 / 111.
+constexpr SlabTimes kBwd64{11.2f, 3.56f, 4.1f, 4.74f, 0.502f, 2, 350, 35.0e-3f, 21.4f, 4.83f, 27.3f, 21.2e-3f};
+// 48 dims 33 heads T = 1024 163 / 212, 48 heads 247 / 230; 57 heads T = 333 47 / 71, 152 heads 122 / 102.
+constexpr SlabTimes kBwd32{4.41f, 4.15f, 3.87f, 3.91f, 0.573f, 2, 350, 32.0e-3f, 6.31f, 12.2f, 14.6f, 25.2e-3f};
+// 16 heads of 128 T = 1024 229 / 330, 33 heads 445 / 340; 40 heads T = 640 239 / 218.
+constexpr SlabTimes kBwd128{4.18f, 5.71f, 5.63f, 5.8f, 0.714f, 1, 250, 89.0e-3f, 0.04f, 20.4f, 30.0f, 59.7e-3f};
+// Heads of 64 up to 128 rows, against the recomputing dk/dv kernel (short_heads_us):
+// 96 heads T = 128 26 / 36, 160 heads 39 / 38; 240 heads T = 64 27 / 25; 270 heads T = 65 39 / 52.
+constexpr SlabTimes kBwdShort{4.0f, 5.7f, 6.5f, 4.4f, 0.5f, 2, 350, 0, 0, 0, 0, 0};
 
 double tiles_of(int B, int H, int nqt) { return 0.5 * B * H * nqt * (nqt + 1); }
 
-bool slab_wins(const SlabTimes &t, double tiles, int nqt) {
-    const double slab = t.fixed + tiles * (tiles < t.r2_from ? t.one : t.two);
-    return slab < std::max<double>(t.chain0 + t.chain * nqt, t.sum0 + t.sum * tiles);
+const SlabTimes &fwd_times(int D) { return D > kDPad ? kFwd128 : D == kDPad ? kFwd64 : kFwd32; }
+const SlabTimes &bwd_times(int D) { return D > kDPad ? kBwd128 : D == kDPad ? kBwd64 : kBwd32; }
+
+int blocks_per_slab(const SlabTimes &t, int B, int H, int nqt) { return tiles_of(B, H, nqt) < t.r2_from ? 1 : 2; }
+
+// slabs: of one head (and kind); wg: workgroups a slab, one in the forward, two in the backward;
+// blocks: on the other side of the last slab (64 keys in the forward, 16 rows in the backward).
+double slab_us(const SlabTimes &t, int R, double slabs, int wg, int heads, int blocks, double tiles) {
+    const double rounds = wg * slabs * heads / (256.0 * t.resident);
+    const double steps = std::max(1.0, blocks / 8.0 + 0.5);
+    const double round = R == 1 ? t.one * steps : t.start2 + t.two * steps;
+    return t.fixed + std::max((rounds + t.tail * (std::ceil(rounds) - rounds)) * round, t.per_tile * tiles);
 }
 
-int blocks_per_slab(const BwdParams &p) {
-    const SlabTimes &t = p.D > kDPad ? kBwd128 : p.D == kDPad ? kBwd64 : kBwd32;
-    return tiles_of(p.B, p.H, p.nqt) < t.r2_from ? 1 : 2;
+double tiled_us(const SlabTimes &t, double tiles, int nqt) {
+    return std::max<double>(t.chain0 + t.chain * nqt, t.sum0 + t.sum * tiles);
+}
+
+// The recomputing dk/dv kernel runs a workgroup per head, in rounds of 256: T = 16 17, 40 22, 64 24, 65 28, 100 35,
+// 128 36 us, two rounds 25 to 67.
+double short_heads_us(int T, int heads) {
+    return (14.5 + 2.75 * ((T + kBlock - 1) / kBlock)) * (0.25 + 0.75 * ((heads + 255) / 256));
 }
 
 template <int R>
@@ -594,32 +626,37 @@ void run_bwd(const BwdParams &p, hipStream_t stream) {
 bool fwd_slab(const FwdParams &p) {
     if (!p.vec || p.qp != nullptr || p.D > 2 * kDPad || !rows_fit(p.T, p.D, {p.q.st, p.k.st, p.v.st})) return false;
     if (p.D == kDPad && p.nqt <= kShortHeadTiles) return false;  // the short-head kernels
-    return slab_wins(p.D > kDPad ? kFwd128 : p.D == kDPad ? kFwd64 : kFwd32, tiles_of(p.B, p.H, p.nqt), p.nqt);
+    const SlabTimes &t = fwd_times(p.D);
+    const int R = blocks_per_slab(t, p.B, p.H, p.nqt), slabs = (p.T + R * kBlock - 1) / (R * kBlock);
+    const double tiles = tiles_of(p.B, p.H, p.nqt);
+    return slab_us(t, R, slabs, 1, p.B * p.H, p.nqt, tiles) < tiled_us(t, tiles, p.nqt);
 }
 
 bool bwd_slab(const BwdParams &p) {
     if (!p.vec || p.D > 2 * kDPad || !rows_fit(p.T, p.D, {p.q.st, p.k.st, p.v.st, p.o.st, p.dout.st})) return false;
+    const SlabTimes &t = bwd_times(p.D);
+    const int R = blocks_per_slab(t, p.B, p.H, p.nqt), heads = p.B * p.H, blocks = (p.T + kBlock - 1) / kBlock;
     const double tiles = tiles_of(p.B, p.H, p.nqt);
-    // Short heads of 64: the recomputing dk/dv kernel runs a workgroup per head, about 30 us a round of 256
-    // (96 heads: T = 128 26 / 36, T = 60 14 / 25; 8 heads T = 100 8 / 32; 200 heads T = 128 56 / 45).
-    if (p.D == kDPad && p.nqt <= kShortHeadTiles) return 8 + 62.5e-3 * tiles < 30.0 * ((p.B * p.H + 255) / 256);
-    return slab_wins(p.D > kDPad ? kBwd128 : p.D == kDPad ? kBwd64 : kBwd32, tiles, p.nqt);
+    if (p.D == kDPad && p.nqt <= kShortHeadTiles)  // few blocks: the last slab's empty half counts
+        return slab_us(kBwdShort, R, static_cast<double>(blocks) / R, 2, heads, blocks, tiles) <
+               short_heads_us(p.T, heads);
+    return slab_us(t, R, (blocks + R - 1) / R, 2, heads, blocks, tiles) < tiled_us(t, tiles, p.nqt);
 }
 
 int slab_count(const BwdParams &p) {
-    const int rows = blocks_per_slab(p) * kBlock;
+    const int rows = blocks_per_slab(bwd_times(p.D), p.B, p.H, p.nqt) * kBlock;
     return (p.T + rows - 1) / rows;
 }
 
 void launch_attn_fwd_slab(const FwdParams &p, hipStream_t stream) {
-    if (p.D > kDPad && tiles_of(p.B, p.H, p.nqt) >= kFwd128.r2_from)
+    if (p.D > kDPad && blocks_per_slab(fwd_times(p.D), p.B, p.H, p.nqt) == 2)
         run_fwd<2>(p, stream);
     else
         run_fwd<1>(p, stream);
 }
 
 void launch_attn_bwd_slab(const BwdParams &p, hipStream_t stream) {
-    if (blocks_per_slab(p) == 1)
+    if (blocks_per_slab(bwd_times(p.D), p.B, p.H, p.nqt) == 1)
         run_bwd<1>(p, stream);
     else
         run_bwd<2>(p, stream);

@@ -317,6 +317,11 @@ long long gptc_decode_noalloc_scratch_floats(void);
  * and [6,7] dq kernels.  They stay registered until the next call;
  * events == NULL stops the recording.  For per-kernel timing.
  *
+ * gptc_attention_slabs(B, T, C, n_heads): the kernels that a shape's calls run
+ *   with 16-byte aligned buffers in the compact cache layout: bit 0 set, the
+ *   forward runs the slab kernels (csrc/attn_slab.hip), bit 1 the backward;
+ *   else the kernels on 64- and 128-row blocks.  Decided on the host; no device
+ *   is needed.
  * gptc_attention_state_floats(B, T, C, n_heads): floats of the 1-D cache[3]
  * that the compact layout's forward expects (and otherwise re-points), so
  * that a layer can allocate it once at the right size.
@@ -370,6 +375,7 @@ void gptc_argmax_cuda(const tensor_t *logits, tensor_t *ids);
 void *gptc_stream(void);
 void gptc_set_kernel_events(void **events, int n);
 long long gptc_attention_state_floats(int B, int T, int C, int n_heads);
+int gptc_attention_slabs(int B, int T, int C, int n_heads);
 
 /*
  * gptc_attention_set_state_limit(floats): no counterpart in gpt.c.  The

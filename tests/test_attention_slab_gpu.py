@@ -122,8 +122,8 @@ def prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift):
 
 @pytest.mark.parametrize("B,T,C,H,shift", [
     (4, 333, 768, 12, 0), (2, 1000, 768, 12, 0), (1, 650, 1600, 25, 0),   # heads of 64
-    (2, 1000, 960, 20, 0), (5, 200, 384, 24, 0),                          # of 48 and 16
-    (5, 208, 1536, 16, 0), (8, 200, 1280, 10, 0),                         # of 96 and 128
+    (2, 1000, 1056, 22, 0), (5, 200, 480, 30, 0),                         # of 48 and 16
+    (5, 333, 1152, 12, 0), (5, 200, 1920, 15, 0),                         # of 96 and 128
     (2, 140, 128, 2, 1), (1, 333, 96, 2, 1), (1, 70, 256, 2, 1),          # gradients that are not 16-byte aligned
 ])
 def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
@@ -131,7 +131,7 @@ def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
     (T ends in the first 16 rows of a half here).  The state is NaN before the forward: a row that it leaves out would
     reach dK and dV as 0 * NaN."""
     print(f"case halves B={B} T={T} C={C} H={H} shift={shift}", flush=True)
-    assert 0 < T % 32 <= 16
+    assert 0 < T % 32 <= 16 and (shift or rt.lib.gptc_attention_slabs(B, T, C, H) == 1)
     prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift)
 
 
