@@ -108,7 +108,8 @@ def test_small_shapes_fwd_bwd(rt, oracle, B, T, C, H):
 
 
 def test_head_size_128_full_length(rt, oracle):
-    """D = 128 over 16 key tiles (T = 1024): the 128-dim forward, dk/dv and dq kernels."""
+    """D = 128 over 16 key tiles (T = 1024): the slab kernels' 128-dim forms with two blocks
+    per wave (the tiled ones: tests/test_attention_tiled_gpu.py)."""
     compare_with_oracle(rt, oracle, 1, 1024, 1024, 8)
 
 
@@ -328,10 +329,9 @@ def test_forward_pool_over_repeated_launches(rt, oracle):
 
 
 def test_split_key_blocks_b1_t1024(rt, oracle):
-    """B*H = 12 heads of T = 1024 fill 96 of the GPU's dk/dv workgroup slots, so
-    each key block with two or more query tiles runs as two workgroups over
-    halves of its query range, adding into dK, dV rows the delta kernel zeroed:
-    oracle parity, and the same bits again (two addends in either order)."""
+    """B*H = 12 heads of T = 1024, which run the slab kernels (cut key blocks of
+    the tiled ones: tests/test_attention_tiled_gpu.py): oracle parity, and the
+    same bits again."""
     compare_with_oracle(rt, oracle, 1, 1024, 768, 12)
     x, dy = qkv_inputs(rt, 1, 1024, 768, 31, 32)
     a = run_layer(rt, x, dy, 12)
@@ -341,8 +341,7 @@ def test_split_key_blocks_b1_t1024(rt, oracle):
 
 
 def test_split_key_blocks_ragged_t(rt, oracle):
-    """Split key blocks when T is not a multiple of the 64-query tile (T = 1000:
-    the last key block and the last query half are partial)."""
+    """The same when T is not a multiple of the 64-query tile (T = 1000)."""
     compare_with_oracle(rt, oracle, 1, 1000, 768, 12)
 
 
@@ -381,7 +380,9 @@ def test_lse_only_state_fwd_bwd(rt, oracle, lse_only_state, B, T, C, H, scratch)
     written to a scratch of every head at once ("whole"), of heads in chunks
     of at most 5 ("chunks": uneven last chunk where B*H is not a multiple of
     5), or, with no scratch ("none"), from a dq kernel that recomputes S and
-    dP too.  Each meets the same tolerance."""
+    dP too.  Each meets the same tolerance.  Shapes of few heads run the slab
+    backward, which needs no scratch (tests/test_attention_tiled_gpu.py has
+    these modes at ragged T with more heads)."""
     n = rt.lib.gptc_attention_state_floats(B, T, C, H)
     assert n < B * H * T * 8 + B * ((T + 63) // 64) * C + 4 * B * ((T + 127) // 128) * C + 4096
     limit = {"whole": -1, "chunks": 5 * ds_floats_per_head(T), "none": 0}[scratch]

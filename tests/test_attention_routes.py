@@ -36,3 +36,12 @@ def test_huge_rows_stay_off_the_slabs(lib):
     """A head's rows past 2^31 bytes (T x 3C floats) are outside a buffer's offsets."""
     assert lib.gptc_attention_slabs(1, 8000, 64 * 400, 400) == 0
     assert lib.gptc_attention_slabs(0, 128, 64, 1) == 0
+
+
+def test_key_blocks_of_twenty_heads_are_cut(lib):
+    """The shape that tests/test_attention_tiled_gpu.py takes for cut key blocks has some (2 workgroups a CU)."""
+    import ctypes
+    buf = [(ctypes.c_int * 20000)() for _ in range(2)]
+    est, nsplit = ctypes.c_double(), ctypes.c_int()
+    assert lib.gptc_attention_key_schedule(20, 16, 2, 32, buf[0], buf[1], 20000, ctypes.byref(est), ctypes.byref(nsplit)) > 0
+    assert nsplit.value > 0

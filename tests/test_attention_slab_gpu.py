@@ -21,20 +21,24 @@ pytestmark = pytest.mark.gpu
     (1, 129, 64, 1), (1, 143, 128, 2), (1, 144, 64, 1), (1, 145, 64, 1), (2, 192, 128, 2), (1, 193, 64, 1),
     (1, 321, 192, 3),
     # two blocks per slab (350 tiles or more)
-    (4, 176, 768, 12), (4, 177, 768, 12), (4, 191, 768, 12), (1, 1024, 192, 3), (1, 1009, 192, 3),
+    # (their forward runs the tiled kernels at T = 176 to 191)
+    (5, 176, 768, 12), (5, 177, 768, 12), (5, 191, 768, 12), (1, 1024, 192, 3), (1, 1009, 192, 3),
     # other head sizes: 4, 16, 36, 60 padded to 64, and 68, 80, 124, 128 to 128
     (2, 33, 8, 2), (1, 100, 16, 1), (2, 70, 72, 2), (3, 200, 120, 2), (2, 48, 136, 2), (2, 161, 160, 2), (1, 97, 248, 2),
     (1, 640, 512, 4), (8, 200, 512, 4), (2, 512, 96, 3),
+    (1, 1009, 1024, 8), (1, 1000, 768, 8),  # from 1000 tiles on heads past 64 run two blocks forward too
 ])
 def test_slabs_against_oracle(rt, oracle, B, T, C, H):
     print(f"case slab B={B} T={T} C={C} H={H}", flush=True)
+    assert rt.lib.gptc_attention_slabs(B, T, C, H) & 2
     compare_with_oracle(rt, oracle, B, T, C, H)
 
 
-@pytest.mark.parametrize("B,T,C,H", [(1, 40, 128, 2), (2, 129, 128, 2), (1, 333, 192, 3), (4, 177, 768, 12)])
+@pytest.mark.parametrize("B,T,C,H", [(1, 40, 128, 2), (2, 129, 128, 2), (1, 333, 192, 3), (5, 177, 768, 12), (1, 1009, 192, 3)])
 def test_slabs_with_qkv_bias(rt, oracle, B, T, C, H):
     """The bias added to the rows and its gradient from the slabs' column sums (one and two blocks per slab)."""
     print(f"case slab bias B={B} T={T} C={C} H={H}", flush=True)
+    assert rt.lib.gptc_attention_slabs(B, T, C, H) & 2
     self_attention_vs_oracle(rt, oracle, B, T, C, H)
 
 

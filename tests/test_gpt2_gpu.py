@@ -154,7 +154,9 @@ def test_self_attention_lse_only_state(rt, oracle, B, T, C, H, scratch):
     bias folded into the recomputing dk/dv kernel and, with a dS scratch of
     every head ("whole") or of 5 heads at a time ("chunks"), into the dq
     kernel that reads it; with no scratch ("none"), dq's bias gradient comes
-    from the recomputing dq kernel's column sums."""
+    from the recomputing dq kernel's column sums.  Shapes that run the slab
+    backward need no scratch: tests/test_attention_tiled_gpu.py has the three
+    modes for the others."""
     nqt = (T + 63) // 64
     limit = {"whole": -1, "chunks": 5 * nqt * (nqt + 1) * 2048, "none": 0}[scratch]
     rt.lib.gptc_attention_set_state_limit(0)
