@@ -1,11 +1,11 @@
 """The compiled-in table of rocBLAS solutions (gpt.c_amd/csrc/gemm_tuned.inc).
 
 Each entry is a column-major rocBLAS problem and a solution index, matched
-field for field against the library's calls (gpt.c_amd/csrc/blas.hip).
+field for field against the sgemm calls (gpt.c_amd/csrc/blas.hip).
 The table is data written by tune_gemm; these checks keep a hand edit or a
-bad merge from naming a problem the library can never issue, two solutions
-for one problem, or two split counts for one weight gradient (the library
-takes the first it finds).  CPU only.
+bad merge from naming a problem that no call can issue, two solutions
+for one problem, or two split counts for one weight gradient (the tuner's
+runs keep the fastest).  CPU only; tests/test_gemm_tuned_gpu.py runs them.
 """
 import os
 import re
@@ -49,9 +49,9 @@ def test_table_keys_are_unique():
 
 
 def test_one_split_count_per_weight_gradient():
-    """gptc_sgemm_wgrad's products: op(A) = N, op(B) = T, C = the (in x out)
-    weight gradient, the reduction over rows cut into `batch` slices (or not,
-    beta = 1 into dW).  One entry per product and total row count."""
+    """Weight gradients: op(A) = N, op(B) = T, C = the (in x out) gradient, the
+    reduction over rows cut into `batch` slices (or not, beta = 1 into it).
+    One entry per product and total row count."""
     per_product = Counter()
     for (ta, tb, m, n, k, lda, ldb, ldc, sa, sb, sc, batch, beta_zero, _), _sol in entries():
         if ta == 0 and tb == 1:

@@ -107,10 +107,10 @@ def test_linear(dev, ops, B, T, in_f, out_f, bias):
 
 @pytest.mark.parametrize("in_f,out_f", [(768, 3072), (3072, 768), (768, 2304)])
 def test_linear_tuned_gemm_shapes(dev, in_f, out_f):
-    """GPT-2's Linear shapes at C3's 8192 rows run rocBLAS solutions from
-    the library's tuned table (csrc/gemm_tuned.inc).  Outputs prefilled with
-    NaN: a solution's first call (validated, then run) must compute every
-    entry and read nothing of C where beta = 0.  Checked against float64
+    """GPT-2's Linear shapes at C3's 8192 rows (the sizes of the tuned rocBLAS
+    table, whose solutions tests/test_gemm_tuned_gpu.py runs; the Linear
+    layers run csrc/gemm_split.hip).  Outputs prefilled with NaN: every entry
+    must be computed and nothing of them read.  Checked against float64
     numpy: y and dx on every 61st row, dW in full (accumulated onto dW0)."""
     print(f"case tuned linear in={in_f} out={out_f}")
     B, T = 8, 1024
