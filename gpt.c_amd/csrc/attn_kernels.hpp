@@ -155,7 +155,7 @@ void launch_attn_fwd(const FwdParams &p, hipStream_t stream, const hipEvent_t *e
 void launch_attn_bwd(const BwdParams &p, hipStream_t stream, const hipEvent_t *ev);
 
 // The slab kernels (attn_slab.hip): whether they run a problem, their launches, and the
-// 16-row slabs of a sequence.  The backward is one launch; with the qkv bias
+// slabs (16 or 32 rows) of a sequence in the backward.  The backward is one launch; with the qkv bias
 // folded in (p.db set), p.dbq_part then takes (B * slab_count(p)) x 3C column sums.
 bool fwd_slab(const FwdParams &p);
 bool bwd_slab(const BwdParams &p);

@@ -33,16 +33,17 @@
 // 8192 3e-7 and 1.6e-6; mean error under 2e-9 at K = 768 and 3072.
 //
 // What bounds it: in a 128 x 128 tile's step a wave issues 48 matrix
-// instructions (1536 cycles) and about 270 vector ones (1080 cycles: 5.5 a float
-// for the split, 64 for the sums); counters at 2000 x 4000 x 1000 read the
-// matrix cores 45 % busy, the vector units 39 %, LDS 23 % with no bank
-// conflicts, at 2.1 GHz.  Moving the next step's split between this step's matrix
-// instructions measured no faster (108.0 against 105.0 us there), nor did
+// instructions (1536 cycles) and about 290 vector ones (1160 cycles: 6.5 a float
+// for the scale and the split, 64 for the sums); counters at 2000 x 4000 x 1000 read the
+// matrix cores 47 % busy (of their cycles, at the 2.1 GHz it runs at), the vector units 43 %,
+// with no bank conflicts.  Moving the next step's split between this step's matrix
+// instructions measured no faster (108.0 against 105.0 us there, before the scale), nor did
 // 256 x 128 tiles (their accumulators spill).  Times in us (GPT-2 small,
 // 8192 rows; rocBLAS's own pick as its caller gets it, this): x W^T to 2304
-// 229 / 189, to 3072 313 / 230, from 3072 to 768 276 / 240, lm_head 4300 / 3700;
-// g W from 2304 225 / 187, from 50257 5800 / 4150; g^T x to 3072 x 768 450 / 240,
-// to 768 x 768 116 / 73.
+// 229 / 202, to 3072 313 / 231, from 3072 to 768 276 / 251, lm_head 4300 / 3870;
+// g W from 2304 225 / 197, from 50257 5800 / 4460; g^T x to 3072 x 768 450 / 250,
+// to 768 x 768 116 / 77.  Without the scale these are 0 to 5 % less (lm_head 3780, g W from
+// 50257 4240): a multiply of each float of the second operand.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>

@@ -208,3 +208,19 @@ def test_tiny_operands_keep_their_bits(rt, case, ex, ew):
     dW, db, dx2 = c(np.zeros((fout, fin), np.float32)), c(np.zeros(fout, np.float32)), c(np.zeros((rows, fin), np.float32))
     rt.lib.linear_backward_cuda_kernel(tg[0], tx[0], tW[0], dW[0], db[0], dx2[0])
     check("dW", np.ldexp(c.get(dW, (fout, fin)), -ex - ew), G.T, np.ldexp(x2.astype(np.float64), -ew))
+
+
+@pytest.mark.parametrize("ex,ew", [(70, 40), (105, -60), (-60, 105), (40, 40)])
+def test_large_operands_and_sums(rt, case, ex, ew):
+    """Floats past 2^104 and sums past 2^80 overflow the split's scale: those blocks are formed in fp32 instead, finite
+    and within what a chain of K fp32 sums shows (2-norm about sqrt(K) 2^-25, 1e-6 here; 2e-6 is asserted)."""
+    print(f"case large ex={ex} ew={ew}", flush=True)
+    rng = np.random.default_rng(8)
+    rows, fin, fout = 1000, 777, 801
+    x, W, g = (np.ldexp(rnd(rng, *s), e) for s, e in (((rows, fin), ex), ((fout, fin), ew), ((rows, fout), ex)))
+    y, dx, _, _ = linear(rt, case(), x, W, np.zeros(fout, np.float32), g)
+    X, W64, G = (np.ldexp(v.astype(np.float64), -e) for v, e in ((x, ex), (W, ew), (g, ex)))
+    for name, got, ref in (("y", y, X @ W64.T), ("dx", dx, G @ W64)):
+        rel = np.linalg.norm(np.ldexp(got, -ex - ew) - ref) / np.linalg.norm(ref)
+        print(f"  {name}: 2-norm {rel:.2e}")
+        assert np.isfinite(got).all() and rel <= 2e-6, name
