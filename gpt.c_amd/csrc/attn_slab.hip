@@ -131,7 +131,12 @@ attn_fwd_slab_kernel(const FwdParams a) {
     const int jq = q0 >> 6;  // the slab's own 64-key tile
     // The backward on 128-key blocks reads P' in halves of 32 queries that start before T, rows
     // past T included: a last slab that ends in the middle of a half writes zeros to the rest of it.
-    const bool fill_half = ((q0 + R * kBlock) & 31) != 0 && q0 + R * kBlock >= T;
+    if (((q0 + R * kBlock) & 31) != 0 && q0 + R * kBlock >= T && a.pp != nullptr)
+        for (int kb32 = w; kb32 <= 2 * jq + 1; kb32 += kSlabWaves) {
+            float *rest = a.pp + ds_block_offset(bh, a.nqt, jq, kb32) + ((q0 & 63) + R * kBlock) * 32;
+            stream_store(reinterpret_cast<f32x4 *>(rest + 4 * lane), zero4());
+            stream_store(reinterpret_cast<f32x4 *>(rest + 4 * lane + 256), zero4());
+        }
 
     const HeadRows<DP> q_rows(a.q.p + b * a.q.sb + h * a.q.sh, T, a.q.st, D);
     const HeadRows<DP> k_rows(a.k.p + b * a.k.sb + h * a.k.sh, T, a.k.st, D);
@@ -210,13 +215,6 @@ attn_fwd_slab_kernel(const FwdParams a) {
                 for (int kb = 0; kb < 4; ++kb)
                     stream_store(reinterpret_cast<f32x4 *>(ptile + (kb >> 1) * kDsBlock + prow + 16 * (kb & 1)),
                                  sc[i][kb]);
-                if (i == R - 1 && fill_half) {
-#pragma unroll
-                    for (int kb = 0; kb < 4; ++kb)
-                        stream_store(reinterpret_cast<f32x4 *>(ptile + (kb >> 1) * kDsBlock + prow + kBlock * 32 +
-                                                               16 * (kb & 1)),
-                                     zero4());
-                }
                 if (g == 0 && my_q < T) a.pm[(static_cast<uint32_t>(bh) * a.nqt + kt) * T + my_q] = m_use;
             }
         }

@@ -33,7 +33,7 @@
 // 8192 3e-7 and 1.6e-6; mean error under 2e-9 at K = 768 and 3072.
 //
 // What bounds it: in a 128 x 128 tile's step a wave issues 48 matrix
-// instructions (1536 cycles) and about 290 vector ones (1160 cycles: 6.5 a float
+// instructions (1536 cycles) and about 280 vector ones (1120 cycles: 6.5 a float
 // for the scale and the split, 64 for the sums); counters at 2000 x 4000 x 1000 read the
 // matrix cores 47 % busy (of their cycles, at the 2.1 GHz it runs at), the vector units 43 %,
 // with no bank conflicts.  Moving the next step's split between this step's matrix
