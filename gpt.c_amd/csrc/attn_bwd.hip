@@ -52,6 +52,11 @@ constexpr int kBwdBQ = 64;   // queries per LDS tile in the dk/dv kernel
 constexpr int kBwdBM = 128;  // queries per dq workgroup (32 per wave)
 constexpr int kBwdBN = 64;   // keys per LDS tile in the dq kernel
 
+// x f, and 0 where f is 0 whatever x is (v_mul_legacy_f32): a half's rows past T have f = 0, and the slab
+// forward leaves their P' as the state held it.
+extern "C" __device__ float gptc_fmul_legacy(float, float) __asm("llvm.amdgcn.fmul.legacy");
+__device__ __forceinline__ float times_or_zero(float x, float f) { return gptc_fmul_legacy(x, f); }
+
 // ---- delta = rowsum(dO o O): 16 lanes per (b, t, h) row, 16 rows per workgroup ----
 template <bool VEC>
 __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const BwdParams a) {
@@ -225,9 +230,9 @@ attn_bwd_dkdv_kernel(const BwdParams a) {
     // P' of one 32-query half, loaded one half ahead of its use: register r
     // holds query 8(r/4) + 4hf + r%4 of the half, key my_k (the accumulator
     // layout of a queries x keys product).  A half is needed when some of
-    // its queries see some of this wave's keys and it starts before T.  The
-    // forward wrote every row of such a half (finite values; rows at or past
-    // T get f = 0), so the loads need no row check.
+    // its queries see some of this wave's keys and it starts before T.  Every
+    // row of such a half lies in the state, and rows at or past T get f = 0
+    // and with it P = 0 (times_or_zero), so the loads need no row check.
     float pbuf[16];
     auto half_needed = [&](int qt, int qb) {
         const int qh0 = qt * kBwdBQ + 32 * qb;
@@ -318,7 +323,7 @@ attn_bwd_dkdv_kernel(const BwdParams a) {
                     for (int g = 0; g < 4; ++g) {
                         const f32x4 f4 = *reinterpret_cast<const f32x4 *>(&f_w[32 * qb + 8 * g + 4 * hf]);
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) s[4 * g + c] = pbuf[4 * g + c] * f4[c];  // P
+                        for (int c = 0; c < 4; ++c) s[4 * g + c] = times_or_zero(pbuf[4 * g + c], f4[c]);  // P
                     }
                 }
             }
@@ -757,7 +762,7 @@ attn_bwd_dkdv_dma_kernel(const BwdParams a) {
                     for (int g = 0; g < 4; ++g) {
                         const f32x4 f4 = *reinterpret_cast<const f32x4 *>(&f_w[32 * qb + 8 * g + 4 * hf]);
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) s[4 * g + c] = pbuf[4 * g + c] * f4[c];  // P
+                        for (int c = 0; c < 4; ++c) s[4 * g + c] = times_or_zero(pbuf[4 * g + c], f4[c]);  // P
                     }
                 }
             }

@@ -15,8 +15,8 @@
 // half dK and dV of a slab of keys; both recompute P from the log-sum-exp and
 // delta = rowsum(dO o O) from the rows at hand: seven products instead of four,
 // but no chain of three launches and no P' or dS through memory.  The longest slabs
-// come first.  (The forward still writes P' and its maxima: a backward that
-// these kernels do not serve reads them.)
+// come first.  (The forward still writes P' and its maxima, up to the last slab's
+// end: a backward that these kernels do not serve reads them.)
 //
 // fp32 on v_mfma_f32_16x16x4_f32 throughout, operand layouts as in
 // attn_common.hpp.  What bounds them: in the backward a wave loads 20 rows of 1 KB
@@ -129,14 +129,6 @@ attn_fwd_slab_kernel(const FwdParams a) {
     const int b = bh / a.H, h = bh - b * a.H;
     const int q0 = ((T + R * kBlock - 1) / (R * kBlock) - 1 - rank) * R * kBlock;  // the longest slabs first
     const int jq = q0 >> 6;  // the slab's own 64-key tile
-    // The backward on 128-key blocks reads P' in halves of 32 queries that start before T, rows
-    // past T included: a last slab that ends in the middle of a half writes zeros to the rest of it.
-    if (((q0 + R * kBlock) & 31) != 0 && q0 + R * kBlock >= T && a.pp != nullptr)
-        for (int kb32 = w; kb32 <= 2 * jq + 1; kb32 += kSlabWaves) {
-            float *rest = a.pp + ds_block_offset(bh, a.nqt, jq, kb32) + ((q0 & 63) + R * kBlock) * 32;
-            stream_store(reinterpret_cast<f32x4 *>(rest + 4 * lane), zero4());
-            stream_store(reinterpret_cast<f32x4 *>(rest + 4 * lane + 256), zero4());
-        }
 
     const HeadRows<DP> q_rows(a.q.p + b * a.q.sb + h * a.q.sh, T, a.q.st, D);
     const HeadRows<DP> k_rows(a.k.p + b * a.k.sb + h * a.k.sh, T, a.k.st, D);

@@ -130,10 +130,10 @@ def prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift):
     (5, 333, 1152, 12, 0), (5, 200, 1920, 15, 0),                         # of 96 and 128
     (2, 140, 128, 2, 1), (1, 333, 96, 2, 1), (1, 70, 256, 2, 1),          # gradients that are not 16-byte aligned
 ])
-def test_stored_probabilities_are_whole_halves(rt, oracle, B, T, C, H, shift):
+def test_stored_probabilities_past_the_last_row(rt, oracle, B, T, C, H, shift):
     """A backward that the slabs do not serve reads the forward's P' in halves of 32 queries, rows past T among them
-    (T ends in the first 16 rows of a half here).  The state is NaN before the forward: a row that it leaves out would
-    reach dK and dV as 0 * NaN."""
+    that a slab of 16 rows does not write (T ends in the first 16 rows of a half here).  The state is NaN before the
+    forward: those rows must not reach dK and dV as 0 * NaN."""
     print(f"case halves B={B} T={T} C={C} H={H} shift={shift}", flush=True)
     assert 0 < T % 32 <= 16 and (shift or rt.lib.gptc_attention_slabs(B, T, C, H) == 1)
     prefilled_state_vs_oracle(rt, oracle, B, T, C, H, shift)
