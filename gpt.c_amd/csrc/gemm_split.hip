@@ -38,7 +38,9 @@
 // matrix cores 47 % busy (of their cycles, at the 2.1 GHz it runs at), the vector units 43 %,
 // with no bank conflicts.  Moving the next step's split between this step's matrix
 // instructions measured no faster (108.0 against 105.0 us there, before the scale), nor did
-// 256 x 128 tiles (their accumulators spill).  Times in us (GPT-2 small,
+// 256 x 128 tiles (their accumulators spill); forming the parts' rests with
+// v_dot2_f32_bf16 (exact, 215 vector instructions a step) is slower (block of 8 x 1024
+// tokens, step 2.98 against 2.89 ms).  Times in us (GPT-2 small,
 // 8192 rows; rocBLAS's own pick as its caller gets it, this): x W^T to 2304
 // 229 / 202, to 3072 313 / 231, from 3072 to 768 276 / 251, lm_head 4300 / 3870;
 // g W from 2304 225 / 197, from 50257 5800 / 4460; g^T x to 3072 x 768 450 / 250,
